@@ -135,6 +135,7 @@ enum {
                               // (default: of one-row products only)
     GRX_TUNE_CONF_ATTN_G8,    // 0: the conformer attention's few-row outputs one a thread, not 8 lanes each
     GRX_TUNE_CONF_ATTN_THREADS,  // 256 or 512: threads of the conformer attention's row-a-workgroup launch
+    GRX_TUNE_PROMPT_ROWS,     // 0: whisper prompts decoded token by token
     GRX_TUNE_COUNT
 };
 int grx_tune(int id);
@@ -445,24 +446,32 @@ grx_status grx_gemm_q8_launch(hipStream_t st, const grx_weight *w, const int8_t 
                               const float *bias, float *y, int ldc);
 // Row kernels (rows.hip): LayerNorm + rounding to Q8_0 of `rows` rows of n
 // values (x rows ldx apart) into xq [rows][n], xs [rows][n/32]; and the
-// whisper decoder's embedding rows (token tok[r], position *pos) written to
-// x [rows][n] before the same.
+// whisper decoder's embedding rows (token tok[r], position *pos + r % per:
+// `per` consecutive positions of each stream) written to x [rows][n] before
+// the same.
 grx_status grx_ln_quant_rows(hipStream_t st, const float *x, int ldx, int rows, int n, const float *w,
                              const float *b, int8_t *xq, float *xs);
 grx_status grx_embed_ln_quant_rows(hipStream_t st, const int *tok, const int *pos, const grx_weight *emb,
-                                   const float *pos_emb, float *x, int rows, const float *w, const float *b,
+                                   const float *pos_emb, float *x, int rows, int per, const float *w, const float *b,
                                    int8_t *xq, float *xs);
+
+// Cross-attention of `per` rows of each stream at once (whisper_prompt.hip):
+// q [streams * per][st], outputs rounded to Q8_0.  Only where
+// grx_cross_prompt_ok says so (heads of 64, a row group's scores in LDS).
+bool grx_cross_prompt_ok(int nctx, int hd);
+grx_status grx_cross_prompt(hipStream_t stream, const float *q, const float *ck, const float *cv, int nctx, int st,
+                            int per, int streams, size_t x_stream, int8_t *att_q, float *att_s);
 
 // Epilogues of the matrix-core product (q8_gemm.hip).
 enum { GRX_GEMM_STORE = 0, GRX_GEMM_ADD = 1, GRX_GEMM_AXPY_HALF = 2, GRX_GEMM_SCALE = 3, GRX_GEMM_SILU_Q = 4,
-       GRX_GEMM_GLU = 5 };
+       GRX_GEMM_GLU = 5, GRX_GEMM_GELU_Q = 6 };
 struct GemmOut {
     float *y = nullptr;  // [m][ldc] (STORE writes it, ADD/AXPY_HALF update it)
     int ldc = 0;
     int epi = GRX_GEMM_STORE;
     float scale = 1.0f;     // SCALE
-    int8_t *yq = nullptr;   // SILU_Q: [m][rows] int8
-    float *ys = nullptr;    //         [m][rows/32] scales
+    int8_t *yq = nullptr;   // SILU_Q, GELU_Q: [m][rows] int8
+    float *ys = nullptr;    //                 [m][rows/32] scales
     // [m][rows] floats the K-split product may use to carry each output's
     // ordered chain from one run of blocks to the next when the weight has
     // more blocks than one workgroup holds (few rows only); NULL: none

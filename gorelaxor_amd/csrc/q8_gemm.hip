@@ -30,6 +30,14 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 
+// The epilogues that round their activation to Q8_0: whole 32-row blocks.
+constexpr bool epi_rounds(int epi) { return epi == GRX_GEMM_SILU_Q || epi == GRX_GEMM_GELU_Q; }
+template <int EPI>
+__device__ __forceinline__ float epi_act(float x) {
+    if constexpr (EPI == GRX_GEMM_GELU_Q) return grx_gelu_avx(x);
+    return __fdiv_rn(x, __fadd_rn(grx_exp8(__fsub_rn(0.0f, x)), 1.0f));
+}
+
 // What the epilogue does with each finished output c (GemmOut::epi):
 //   STORE      y = c
 //   ADD        y = y + c                      (kern.Add of the product)
@@ -37,6 +45,8 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 //   SCALE      y = c * scale
 //   SILU_Q     SiLU(c) of the AVX route (c / (EXP8(0 - c) + 1)), rounded to
 //              Q8_0 per 32 outputs into yq [m][rows], ys [m][rows/32]
+//   GELU_Q     geluVec(c) (rows % 32 == 0, so every value takes the AVX
+//              form: kernels_amd64.go:119-129), rounded the same way
 //   GLU        rows paired (grx_glu_row): y [m][rows/2] = a * sigmoid(b)
 //              (the K-split kernel and the one-row GEMV only)
 //
@@ -181,7 +191,7 @@ tail:
         fold(t, 1);
     }
 
-    if constexpr (EPI == GRX_GEMM_SILU_Q) {
+    if constexpr (epi_rounds(EPI)) {
         // The wave's columns are whole Q8_0 blocks (NS even): block j holds
         // columns 16*(2j) + li and 16*(2j+1) + li of the 16 lanes sharing lk,
         // so a row's block maximum is four xor-shuffles within those lanes.
@@ -197,7 +207,7 @@ tail:
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const float x = c[2 * j + h][r];
-                    v[h] = __fdiv_rn(x, __fadd_rn(grx_exp8(__fsub_rn(0.0f, x)), 1.0f));
+                    v[h] = epi_act<EPI>(x);
                 }
                 const float a0 = fabsf(v[0]), a1 = fabsf(v[1]);
                 float amax = a0 > 0.0f ? a0 : 0.0f;
@@ -400,7 +410,7 @@ __global__ __launch_bounds__(64 * ks_max_waves(NS, KB)) void gemm_q8_ks_kernel(
     }
     if (wave != ks - 1) return;
 
-    if constexpr (EPI == GRX_GEMM_SILU_Q) {
+    if constexpr (epi_rounds(EPI)) {
         // the tile's 32 columns are one Q8_0 block (rows % 32 == 0): a row's
         // block maximum is four xor-shuffles among the 16 lanes sharing lk
         static_assert(NS == 2, "rounded output needs whole 32-column blocks per tile");
@@ -412,7 +422,7 @@ __global__ __launch_bounds__(64 * ks_max_waves(NS, KB)) void gemm_q8_ks_kernel(
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const float x = c[h][r];
-                v[h] = __fdiv_rn(x, __fadd_rn(grx_exp8(__fsub_rn(0.0f, x)), 1.0f));
+                v[h] = epi_act<EPI>(x);
             }
             const float a0 = fabsf(v[0]), a1 = fabsf(v[1]);
             float amax = a0 > 0.0f ? a0 : 0.0f;
@@ -771,7 +781,7 @@ gemm_q8_kss_kernel(
     }
     if (wave != ks - 1) return;
 
-    if constexpr (EPI == GRX_GEMM_SILU_Q) {
+    if constexpr (epi_rounds(EPI)) {
         // the tile's 32 columns are one Q8_0 block of the activation row
         // (rows % 32 == 0), spread over the four lanes li, li+16, li+32,
         // li+48: their block maximum is two xor-shuffles
@@ -784,7 +794,7 @@ gemm_q8_kss_kernel(
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float x = c[h][r];
-                v[h][r] = __fdiv_rn(x, __fadd_rn(grx_exp8(__fsub_rn(0.0f, x)), 1.0f));
+                v[h][r] = epi_act<EPI>(x);
                 const float a = fabsf(v[h][r]);
                 amax = a > amax ? a : amax;
             }
@@ -1034,7 +1044,7 @@ __global__ __launch_bounds__(kLdsThreads) void gemm_q8_lds_kernel(const int8_t *
             drow[r] = mb + 32 * wm + 16 * f + 4 * lk + r;
             drow_ok[r] = drow[r] < m;
         }
-        if constexpr (EPI == GRX_GEMM_SILU_Q) {
+        if constexpr (epi_rounds(EPI)) {
             // the wave's 32 columns are one Q8_0 block (rows % 32 == 0)
             const int nr = rows / GRX_QK;
             const int n0 = t0 * 64 + 32 * wn;
@@ -1045,7 +1055,7 @@ __global__ __launch_bounds__(kLdsThreads) void gemm_q8_lds_kernel(const int8_t *
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const float x = c[f][h][r];
-                    v[h] = __fdiv_rn(x, __fadd_rn(grx_exp8(__fsub_rn(0.0f, x)), 1.0f));
+                    v[h] = epi_act<EPI>(x);
                 }
                 const float a0 = fabsf(v[0]), a1 = fabsf(v[1]);
                 float amax = a0 > 0.0f ? a0 : 0.0f;
@@ -1123,12 +1133,12 @@ __global__ __launch_bounds__(kLdsThreads) void gemm_q8_lds_kernel(const int8_t *
 // (16*NS weight rows per wave), NS = 4 once there are plenty.
 int pick_ns(int m, int rows, int epi) {
     const int v = grx_tune(GRX_TUNE_GEMM_NS);
-    if (v == 1 || v == 2 || v == 4) return (epi == GRX_GEMM_SILU_Q && v == 1) ? 2 : v;
+    if (v == 1 || v == 2 || v == 4) return (epi_rounds(epi) && v == 1) ? 2 : v;
     // (measured at 64 and 126 rows: two 16-column tiles per wave win from
     // about 384 of these on, e.g. 126 x 4096 x 1024 14.0 -> 10.0 us)
     const long waves4 = (long)grx_ceil_div(m, 16) * grx_ceil_div(rows, 64);
     int ns = waves4 >= 4096 ? 4 : (waves4 >= 384 ? 2 : 1);
-    if (epi == GRX_GEMM_SILU_Q && ns == 1) ns = 2;
+    if (epi_rounds(epi) && ns == 1) ns = 2;
     return ns;
 }
 
@@ -1150,7 +1160,7 @@ int pick_ns(int m, int rows, int epi) {
 // 8 blocks (8 x 1280 x 5120: 23.6 us on the GEMV, two runs here).  False
 // when a workgroup of ks_max_waves waves cannot hold the weight's blocks.
 bool pick_ks(int m, int nb, int rows, int epi, bool carry, bool sa, bool pro, int *ns, int *kb) {
-    const bool pair = epi == GRX_GEMM_SILU_Q || epi == GRX_GEMM_GLU;  // whole 32-row tiles
+    const bool pair = epi_rounds(epi) || epi == GRX_GEMM_GLU;  // whole 32-row tiles
     const bool few = grx_ceil_div(m, 16) <= 2 && !pair;
     int n, k;
     if (sa) {
@@ -1268,7 +1278,7 @@ void launch_ks_sa(hipStream_t st, const grx_weight *w, const int8_t *xq, const f
 template <int EPI>
 void launch_ks_epi(hipStream_t st, const grx_weight *w, const int8_t *xq, const float *xs, int m, const float *bias,
                    const GemmOut &o, int ns, int kb, int da4, bool sa) {
-    if constexpr (EPI != GRX_GEMM_SILU_Q) {
+    if constexpr (!epi_rounds(EPI)) {
         if (ns == 1) {
             if (kb == 4) return launch_ks_sa<EPI, 1, 4>(st, w, xq, xs, m, bias, o, da4, sa);
             if (kb == 8) return launch_ks_sa<EPI, 1, 8>(st, w, xq, xs, m, bias, o, da4, sa);
@@ -1350,7 +1360,7 @@ RoutePick pick_route(const grx_weight *w, const int8_t *xq, const float *xs, int
     const int kind = grx_tune(GRX_TUNE_GEMM_KERNEL);
     const bool pro = o.x != nullptr;
     RoutePick p{kRouteMfma, 1, 4, 0, false};
-    if (m == 1 && kind < 0 && o.carry == nullptr && o.epi != GRX_GEMM_SCALE && w->nb > 0 &&
+    if (m == 1 && kind < 0 && o.carry == nullptr && o.epi != GRX_GEMM_SCALE && o.epi != GRX_GEMM_GELU_Q && w->nb > 0 &&
         grx_tune(GRX_TUNE_GEMV1) != 0) {
         p.r = kRouteGemv1;
         return p;
@@ -1396,9 +1406,9 @@ bool grx_gemm_q8_fuses(const grx_weight *w, int m, const GemmOut &o) {
 grx_status grx_gemm_q8_launch_ex(hipStream_t st, const grx_weight *w, const int8_t *xq, const float *xs, int m,
                                  const float *bias, const GemmOut &o) {
     if (m <= 0 || w->rows == 0) return GRX_OK;
-    if (o.epi < GRX_GEMM_STORE || o.epi > GRX_GEMM_GLU)
+    if (o.epi < GRX_GEMM_STORE || o.epi > GRX_GEMM_GELU_Q)
         return grx_fail(GRX_EINVAL, "unknown product epilogue %d", o.epi);
-    if ((o.epi == GRX_GEMM_SILU_Q || o.epi == GRX_GEMM_GLU) && w->rows % GRX_QK != 0)
+    if ((epi_rounds(o.epi) || o.epi == GRX_GEMM_GLU) && w->rows % GRX_QK != 0)
         return grx_fail(GRX_ESIZE, "rounded or paired product output needs rows %% 32 == 0 (rows %d)", w->rows);
     const bool fused = fused_parts(o);
     if (fused && !grx_gemm_q8_fuses(w, m, o))
@@ -1453,6 +1463,7 @@ grx_status grx_gemm_q8_launch_ex(hipStream_t st, const grx_weight *w, const int8
             GRX_GEMM_LDS(GRX_GEMM_SCALE)
             GRX_GEMM_LDS(GRX_GEMM_SILU_Q)
             GRX_GEMM_LDS(GRX_GEMM_GLU)
+            GRX_GEMM_LDS(GRX_GEMM_GELU_Q)
         }
 #undef GRX_GEMM_LDS
         GRX_LAUNCHED("gemm_q8_lds_kernel");
@@ -1483,6 +1494,9 @@ grx_status grx_gemm_q8_launch_ex(hipStream_t st, const grx_weight *w, const int8
             case GRX_GEMM_SILU_Q:
                 launch_ks_epi<GRX_GEMM_SILU_Q>(st, w, xq, xs, m, bias, o, 2, p.kb, p.da4, p.sa);
                 break;
+            case GRX_GEMM_GELU_Q:
+                launch_ks_epi<GRX_GEMM_GELU_Q>(st, w, xq, xs, m, bias, o, 2, p.kb, p.da4, p.sa);
+                break;
         }
         GRX_LAUNCHED("gemm_q8_ks_kernel");
         return GRX_OK;
@@ -1511,6 +1525,12 @@ grx_status grx_gemm_q8_launch_ex(hipStream_t st, const grx_weight *w, const int8
                 GRX_GEMM_GO(GRX_GEMM_SILU_Q, 4, GRX_GEMM_U4);
             else
                 GRX_GEMM_GO(GRX_GEMM_SILU_Q, 2, GRX_GEMM_U2);
+            break;
+        case GRX_GEMM_GELU_Q:
+            if (ns == 4)
+                GRX_GEMM_GO(GRX_GEMM_GELU_Q, 4, GRX_GEMM_U4);
+            else
+                GRX_GEMM_GO(GRX_GEMM_GELU_Q, 2, GRX_GEMM_U2);
             break;
     }
 #undef GRX_GEMM_CASE

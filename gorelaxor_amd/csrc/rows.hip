@@ -66,18 +66,18 @@ __global__ __launch_bounds__(kThreads) void ln_quant_rows_kernel(const float *__
     quant_lds_row(row, n, xq + (size_t)r * n, xs + (size_t)r * (n / 32));
 }
 
-// Row r = stream r: x[r] = tokEmb.row(tok[r]) + decPos[*pos] (whisper/
-// decoder.go:42-46; the embedding row widened from its Q8_0 tile layout,
+// Row r: x[r] = tokEmb.row(tok[r]) + decPos[*pos + r % per] (whisper/
+// decoder.go:42-46; `per` consecutive positions of each stream, 1 in a step; the embedding row widened from its Q8_0 tile layout,
 // d*q then + pos unfused), stored as the residual stream, then LayerNorm
 // and rounding as above.
 __global__ __launch_bounds__(kThreads) void embed_ln_quant_kernel(
     const int *__restrict__ tok, const int *__restrict__ pos, const int8_t *__restrict__ emb_qs,
     const uint16_t *__restrict__ emb_ds, int nb, const float *__restrict__ pos_emb, float *__restrict__ x,
-    const float *__restrict__ w, const float *__restrict__ b, int8_t *__restrict__ xq, float *__restrict__ xs) {
+    int per, const float *__restrict__ w, const float *__restrict__ b, int8_t *__restrict__ xq, float *__restrict__ xs) {
     extern __shared__ __align__(16) float row[];
     __shared__ double red[48];  // ln_block_reduce
     const int r = blockIdx.x, n = nb * GRX_QK;
-    const int t = tok[r], p = *pos;
+    const int t = tok[r], p = *pos + r % per;
     const int etile = t >> 6, elane = t & 63;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         const int bk = i >> 5, h = (i >> 4) & 1, e = i & 15;
@@ -103,11 +103,11 @@ grx_status grx_ln_quant_rows(hipStream_t st, const float *x, int ldx, int rows, 
 }
 
 grx_status grx_embed_ln_quant_rows(hipStream_t st, const int *tok, const int *pos, const grx_weight *emb,
-                                   const float *pos_emb, float *x, int rows, const float *w, const float *b,
+                                   const float *pos_emb, float *x, int rows, int per, const float *w, const float *b,
                                    int8_t *xq, float *xs) {
     if (rows <= 0) return GRX_OK;
     embed_ln_quant_kernel<<<rows, kThreads, (size_t)emb->nb * GRX_QK * 4, st>>>(tok, pos, emb->qs, emb->ds, emb->nb,
-                                                                              pos_emb, x, w, b, xq, xs);
+                                                                              pos_emb, x, per, w, b, xq, xs);
     GRX_LAUNCHED("embed_ln_quant_kernel");
     return GRX_OK;
 }

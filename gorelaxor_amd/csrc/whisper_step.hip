@@ -113,9 +113,10 @@ __device__ __forceinline__ void self_attn_small(float *sm, const float *q, const
     }
 }
 
-// Causal self-attention of one head (blockIdx.x) of one stream (blockIdx.y,
-// its cache kv_stream floats after the previous stream's) over the pos+1
-// cached positions (decoder.go:70-87): scores dotF32Go(q, k_j)*sc, softmax, and
+// Causal self-attention of one head (blockIdx.x) of one row (blockIdx.y: row
+// y % per of stream y / per, at position pos + y % per; per = 1 in a step;
+// the stream's cache kv_stream floats after the previous stream's) over the
+// cached positions up to the row's own (decoder.go:70-87): scores dotF32Go(q, k_j)*sc, softmax, and
 // out[d] += p_j * v_j[d] in position order, unfused.  With QOUT (head_dim a
 // multiple of 32) the head's outputs are also rounded to Q8_0 for the out
 // projection.  Heads of 64 over at most kSmallN positions take the
@@ -124,16 +125,17 @@ template <bool QOUT>
 __global__ __launch_bounds__(kAttnThreads) void self_attn_kernel(
     const float *__restrict__ q, const float *__restrict__ kc, const float *__restrict__ vc,
     const int *__restrict__ pos, int st, int hd, float sc, int rc, size_t kv_stream, float *__restrict__ att,
-    int8_t *__restrict__ att_q, float *__restrict__ att_s, int ctx_rows) {
+    int8_t *__restrict__ att_q, float *__restrict__ att_s, int ctx_rows, int per) {
     extern __shared__ __align__(16) float sm[];
-    const int h = blockIdx.x, tid = threadIdx.x, sm_ = blockIdx.y;  // head, stream
-    const int n = *pos + 1;
+    const int h = blockIdx.x, tid = threadIdx.x, sm_ = blockIdx.y;  // head, row
+    const size_t kv0 = (size_t)(sm_ / per) * kv_stream;
+    const int n = *pos + sm_ % per + 1;
     if (hd == kSmallHd && n <= kSmallN) {
         // thread j's K and V row j (many lanes loading one repeated row
         // measured far slower than leaving them out)
         const int j = min(min(tid, n - 1), ctx_rows - 1);
-        const float4 *kr = reinterpret_cast<const float4 *>(kc + sm_ * kv_stream + (size_t)j * st + h * kSmallHd);
-        const float4 *vr = reinterpret_cast<const float4 *>(vc + sm_ * kv_stream + (size_t)j * st + h * kSmallHd);
+        const float4 *kr = reinterpret_cast<const float4 *>(kc + kv0 + (size_t)j * st + h * kSmallHd);
+        const float4 *vr = reinterpret_cast<const float4 *>(vc + kv0 + (size_t)j * st + h * kSmallHd);
         float4 kv[kSmallHd / 4], vv[kSmallHd / 4];
         if (tid < n) {  // lanes past n load nothing
 #pragma unroll
@@ -151,8 +153,8 @@ __global__ __launch_bounds__(kAttnThreads) void self_attn_kernel(
     }
     float *part = sm, *s = sm + 32, *vl = sm + 32 + ((n + 3) & ~3);
     q += (size_t)sm_ * st;
-    kc += sm_ * kv_stream;
-    vc += sm_ * kv_stream;
+    kc += kv0;
+    vc += kv0;
     att += (size_t)sm_ * st;
     if constexpr (QOUT) {
         att_q += (size_t)sm_ * st;
@@ -850,6 +852,31 @@ __global__ void cross_layout_kernel(const float *__restrict__ k, const float *__
     cv[((size_t)h * hd + d) * nctx + t] = v[i];
 }
 
+// A prompt's q | k | v rows [row][3 st] (row r: position *pos + r % per of
+// stream r / per): q into its own rows, k and v into the caches.
+__global__ __launch_bounds__(256) void prompt_kv_kernel(const float *__restrict__ qkv, const int *__restrict__ pos,
+                                                        int st, int per, size_t kv_stream, float *__restrict__ q,
+                                                        float *__restrict__ kc, float *__restrict__ vc) {
+    const int r = blockIdx.x, n4 = st / 4;  // st % 32 == 0
+    const float4 *s = reinterpret_cast<const float4 *>(qkv + (size_t)r * 3 * st);
+    const size_t row = (size_t)(r / per) * kv_stream + (size_t)(*pos + r % per) * st;
+    float4 *dst[3] = {reinterpret_cast<float4 *>(q + (size_t)r * st), reinterpret_cast<float4 *>(kc + row),
+                      reinterpret_cast<float4 *>(vc + row)};
+    for (int i = threadIdx.x; i < n4; i += blockDim.x)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) dst[k][i] = s[k * n4 + i];
+}
+
+// A pass's last rows (row per - 1 of each stream) for the logits, and the
+// position moved on.
+__global__ __launch_bounds__(256) void prompt_last_kernel(const float *__restrict__ x, int st, int per,
+                                                          float *__restrict__ out, int *__restrict__ pos, int add) {
+    const float4 *s = reinterpret_cast<const float4 *>(x + ((size_t)blockIdx.x * per + per - 1) * st);
+    for (int i = threadIdx.x; i < st / 4; i += blockDim.x)
+        reinterpret_cast<float4 *>(out + (size_t)blockIdx.x * st)[i] = s[i];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *pos += add;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------- host side
@@ -882,6 +909,11 @@ struct grx_whisper {
     unsigned long long *keys = nullptr;  // argmax keys, [vocabulary tiles][streams]
     unsigned int *counter = nullptr;
     int *tok = nullptr, *pos = nullptr, *hist = nullptr;
+    // a prompt's rows (grown to the largest prompt: pr_cap rows)
+    int pr_cap = 0;
+    int *pr_tok = nullptr;
+    float *pr_x = nullptr, *pr_y = nullptr, *pr_q = nullptr, *pr_as = nullptr, *pr_fs = nullptr;
+    int8_t *pr_aq = nullptr, *pr_fq = nullptr;
     float *xenc = nullptr, *xk_tmp = nullptr, *xv_tmp = nullptr;  // cross K/V precompute staging
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -1093,17 +1125,61 @@ grx_status launch_qkv_attn(hipStream_t stream, const GemvArgs &a, int nh, float 
     return GRX_OK;
 }
 
-// The launches of one decode step on stream st.
-grx_status enqueue_step(grx_whisper *m, hipStream_t stream) {
+// Several streams: a product's prologue builds each stream's row with one
+// wave per row (rows up to 1280 values); wider rows are LayerNorm'd and
+// rounded once by a row kernel and read pre-rounded (GRX_FUSE_LN=0 takes
+// that route for every width).
+bool sep_ln(const grx_whisper *m) { return m->S > 1 && (m->hp.n_state > 1280 || tuned_off(GRX_TUNE_FUSE_LN)); }
+
+// The end of a step, of the S rows in x: LN -> logits = tokEmb . h ->
+// argmax; the last workgroup writes the tokens and moves the position on.
+grx_status enqueue_logits(grx_whisper *m, hipStream_t stream) {
     const grx_whisper_hparams &hp = m->hp;
-    const int st = hp.n_state, nh = hp.n_head, hd = st / nh, nctx = hp.n_audio_ctx;
+    const int st = hp.n_state, S = m->S;
+    GemvArgs a = gemv_args(m->tok_emb);
+    a.streams = S > 1;
+    a.kv_stream = (size_t)hp.n_text_ctx * st;
+    a.hist_stream = hp.n_text_ctx;
+    a.cacheable = 0;  // 26.5 MB streamed once per step: non-temporal loads
+    a.x = m->x;
+    a.lda = st;
+    a.ln_w = m->dec_ln_w;
+    a.ln_b = m->dec_ln_b;
+    a.y = m->logits;
+    a.ldc = hp.n_vocab;
+    // per-workgroup argmax keys and a one-workgroup end of step (no
+    // contended atomics); ARGMAX_ATOMIC tuned to 1 takes the atomic form
+    const bool atomic_form = grx_tune(GRX_TUNE_ARGMAX_ATOMIC) == 1;
+    a.amax = m->amax;
+    if (atomic_form)
+        a.counter = m->counter;
+    else
+        a.keys = m->keys;
+    a.tok_w = m->tok;
+    a.pos = m->pos;
+    a.pos_w = m->pos;
+    a.hist = m->hist;
+    if (sep_ln(m)) {
+        a.xq = m->ln_q;
+        a.xs = m->ln_s;
+        const grx_status s = grx_ln_quant_rows(stream, m->x, st, S, st, m->dec_ln_w, m->dec_ln_b, m->ln_q, m->ln_s);
+        if (s != GRX_OK) return s;
+        return grx_gemv_launch(stream, S, GRX_PRO_PREQ, GRX_EPI_ARGMAX, a, 0);
+    }
+    return grx_gemv_launch(stream, S, GRX_PRO_LN, GRX_EPI_ARGMAX, a, 0);
+}
+
+// The self-attention of `per` rows of each stream (1 in a step), their q
+// rows [S * per][st] given and their keys and values in the cache.
+grx_status launch_self_attn(grx_whisper *m, hipStream_t stream, const WLayer &L, const float *q, int per, float *att,
+                            int8_t *att_q, float *att_s) {
+    const grx_whisper_hparams &hp = m->hp;
+    const int st = hp.n_state, nh = hp.n_head, hd = st / nh;
     const float sc = (float)(1.0 / sqrt((double)hd));
-    const bool qatt = hd % 32 == 0;  // attention outputs are whole Q8_0 blocks per head
-    grx_status s;
     const int rc = std::max(1, std::min(hp.n_text_ctx, (48 * 1024) / (hd * 4)));
-    size_t attn_smem = (32 + (((size_t)hp.n_text_ctx + 3) & ~(size_t)3) + (size_t)rc * hd) * 4;
+    size_t smem = (32 + (((size_t)hp.n_text_ctx + 3) & ~(size_t)3) + (size_t)rc * hd) * 4;
     if (hd == kSmallHd) {
-        attn_smem = std::max(attn_smem, kSmallLds * 4);
+        smem = std::max(smem, kSmallLds * 4);
         static bool raised = false;  // set by the eager step that precedes any capture
         if (!raised) {
             raised = true;
@@ -1113,6 +1189,133 @@ grx_status enqueue_step(grx_whisper *m, hipStream_t stream) {
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kSmallLds * 4)));
         }
     }
+    const dim3 grid(nh, m->S * per);
+    const size_t kv_stream = (size_t)hp.n_text_ctx * st;
+    if (hd % 32 == 0)  // whole Q8_0 blocks per head
+        self_attn_kernel<true><<<grid, kAttnThreads, smem, stream>>>(q, L.self_k, L.self_v, m->pos, st, hd, sc, rc,
+                                                                     kv_stream, att, att_q, att_s, hp.n_text_ctx, per);
+    else
+        self_attn_kernel<false><<<grid, kAttnThreads, smem, stream>>>(q, L.self_k, L.self_v, m->pos, st, hd, sc, rc,
+                                                                      kv_stream, att, nullptr, nullptr, hp.n_text_ctx,
+                                                                      per);
+    GRX_LAUNCHED("self_attn_kernel");
+    return GRX_OK;
+}
+
+// Rows of a prompt decoded in one pass (all streams together; the workspace
+// is sized for them), and the fewest positions that take it: a pass is about
+// 80 launches of ~5 us at base.en, a step 0.22 ms (a 4-token prompt and 96
+// steps: 22.12 ms as steps, 21.93 with the prompt in a pass; 8 streams of
+// large-v3-turbo 48.7 and 47.2).
+constexpr int kPromptRows = 256;
+constexpr int kPromptMin = 3;
+
+// Whether prompts run as rows of many-row products (heads of 64, a row
+// group's cross scores in LDS); else, or tuned off, token by token.
+bool prompt_rows_ok(const grx_whisper *m) {
+    const grx_whisper_hparams &hp = m->hp;
+    return !tuned_off(GRX_TUNE_PROMPT_ROWS) && grx_cross_prompt_ok(hp.n_audio_ctx, hp.n_state / hp.n_head);
+}
+
+grx_status prompt_alloc(grx_whisper *m) {
+    if (m->pr_cap > 0) return GRX_OK;
+    const size_t R = kPromptRows, st = m->hp.n_state;
+    grx_status s;
+    if (!m->pr_tok && (s = dev_alloc_t(m, (size_t)m->S * m->hp.n_text_ctx, &m->pr_tok)) != GRX_OK) return s;
+    if (!m->pr_x && (s = dev_alloc_t(m, R * st, &m->pr_x)) != GRX_OK) return s;
+    if (!m->pr_y && (s = dev_alloc_t(m, R * 3 * st, &m->pr_y)) != GRX_OK) return s;
+    if (!m->pr_q && (s = dev_alloc_t(m, R * st, &m->pr_q)) != GRX_OK) return s;
+    if (!m->pr_aq && (s = dev_alloc_t(m, R * st, &m->pr_aq)) != GRX_OK) return s;
+    if (!m->pr_as && (s = dev_alloc_t(m, R * st / 32, &m->pr_as)) != GRX_OK) return s;
+    if (!m->pr_fq && (s = dev_alloc_t(m, R * 4 * st, &m->pr_fq)) != GRX_OK) return s;
+    if (!m->pr_fs && (s = dev_alloc_t(m, R * 4 * st / 32, &m->pr_fs)) != GRX_OK) return s;
+    m->pr_cap = kPromptRows;
+    return GRX_OK;
+}
+
+// `per` prompt positions of every stream at once, from the position the
+// device holds: the step's graph with S * per rows in every product
+// (decoder.go:33-140 takes the prompt's rows together too).  Every output
+// of a product, and every row's attention, sees the same operations in the
+// same order as in a step, so the bits are the step's.
+//
+// A prompt position decoded as a step costs the step's chain of 44 dependent
+// launches and every weight once more; as rows they share both (base.en, 187
+// tokens with the window's cross keys and values: 42.5 ms token by token,
+// 1.1 ms in one pass, of it 0.28 ms cross-attention and 0.12 ms
+// self-attention).
+grx_status enqueue_prompt(grx_whisper *m, hipStream_t stream, const int *tok, int per, bool last) {
+    const grx_whisper_hparams &hp = m->hp;
+    const int st = hp.n_state, nctx = hp.n_audio_ctx, S = m->S, R = S * per;
+    const size_t kv_stream = (size_t)hp.n_text_ctx * st, x_stream = (size_t)nctx * st;
+    grx_status s;
+    auto gemm = [&](const grx_weight *w, const int8_t *xq, const float *xs, const float *b, float *y, int ldc, int epi) {
+        GemmOut o;
+        o.y = y;
+        o.ldc = ldc;
+        o.epi = epi;
+        o.yq = m->pr_fq;
+        o.ys = m->pr_fs;
+        return grx_gemm_q8_launch_ex(stream, w, xq, xs, R, b, o);
+    };
+    auto ln = [&](const float *w, const float *b) {
+        return grx_ln_quant_rows(stream, m->pr_x, st, R, st, w, b, m->pr_aq, m->pr_as);
+    };
+    for (int li = 0; li < hp.n_layer; ++li) {
+        const WLayer &L = m->L[li];
+        s = li == 0 ? grx_embed_ln_quant_rows(stream, tok, m->pos, m->tok_emb, m->dec_pos, m->pr_x, R, per,
+                                              L.attn_ln_w, L.attn_ln_b, m->pr_aq, m->pr_as)
+                    : ln(L.attn_ln_w, L.attn_ln_b);
+        if (s != GRX_OK) return s;
+        if ((s = gemm(L.qkv, m->pr_aq, m->pr_as, L.qkv_b, m->pr_y, 3 * st, GRX_GEMM_STORE)) != GRX_OK) return s;
+        prompt_kv_kernel<<<R, 256, 0, stream>>>(m->pr_y, m->pos, st, per, kv_stream, m->pr_q, L.self_k, L.self_v);
+        GRX_LAUNCHED("prompt_kv_kernel");
+        if ((s = launch_self_attn(m, stream, L, m->pr_q, per, m->pr_y, m->pr_aq, m->pr_as)) != GRX_OK) return s;
+        if ((s = gemm(L.o, m->pr_aq, m->pr_as, L.o_b, m->pr_x, st, GRX_GEMM_ADD)) != GRX_OK) return s;
+        if ((s = ln(L.x_ln_w, L.x_ln_b)) != GRX_OK) return s;
+        if ((s = gemm(L.xq, m->pr_aq, m->pr_as, L.xq_b, m->pr_q, st, GRX_GEMM_STORE)) != GRX_OK) return s;
+        if ((s = grx_cross_prompt(stream, m->pr_q, L.cross_k, L.cross_v, nctx, st, per, S, x_stream, m->pr_aq,
+                                  m->pr_as)) != GRX_OK)
+            return s;
+        if ((s = gemm(L.xo, m->pr_aq, m->pr_as, L.xo_b, m->pr_x, st, GRX_GEMM_ADD)) != GRX_OK) return s;
+        if ((s = ln(L.mlp_ln_w, L.mlp_ln_b)) != GRX_OK) return s;
+        if ((s = gemm(L.fc1, m->pr_aq, m->pr_as, L.fc1_b, nullptr, 0, GRX_GEMM_GELU_Q)) != GRX_OK) return s;
+        if ((s = gemm(L.fc2, m->pr_fq, m->pr_fs, L.fc2_b, m->pr_x, st, GRX_GEMM_ADD)) != GRX_OK) return s;
+    }
+    prompt_last_kernel<<<S, 256, 0, stream>>>(m->pr_x, st, per, m->x, m->pos, last ? per - 1 : per);
+    GRX_LAUNCHED("prompt_last_kernel");
+    return last ? enqueue_logits(m, stream) : GRX_OK;
+}
+
+// n prompt positions of every stream (prompts [S][n]) from the position
+// reached, in passes of at most kPromptRows rows.
+grx_status run_prompt(grx_whisper *m, const int32_t *prompts, int n) {
+    const int S = m->S, most = kPromptRows / S;
+    hipStream_t stream = m->ctx->stream;
+    grx_status s = prompt_alloc(m);
+    if (s != GRX_OK) return s;
+    std::vector<int32_t> order;  // each pass's tokens as its rows are
+    order.reserve((size_t)S * n);
+    for (int i = 0; i < n; i += most)
+        for (int k = 0; k < S; ++k)
+            order.insert(order.end(), prompts + (size_t)k * n + i, prompts + (size_t)k * n + std::min(n, i + most));
+    GRX_HIP(hipMemcpyAsync(m->pr_tok, order.data(), order.size() * 4, hipMemcpyHostToDevice, stream));
+    for (int i = 0; i < n; i += most) {
+        const int per = std::min(most, n - i);
+        if ((s = enqueue_prompt(m, stream, m->pr_tok + (size_t)S * i, per, i + per == n)) != GRX_OK) return s;
+        m->pos_host += per;
+    }
+    GRX_HIP(hipStreamSynchronize(stream));  // order is read by the copy
+    return GRX_OK;
+}
+
+// The launches of one decode step on stream st.
+grx_status enqueue_step(grx_whisper *m, hipStream_t stream) {
+    const grx_whisper_hparams &hp = m->hp;
+    const int st = hp.n_state, nh = hp.n_head, hd = st / nh, nctx = hp.n_audio_ctx;
+    const float sc = (float)(1.0 / sqrt((double)hd));
+    const bool qatt = hd % 32 == 0;  // attention outputs are whole Q8_0 blocks per head
+    grx_status s;
     const size_t val_smem = (64 + (size_t)nctx) * 4;
     const int dg = qatt ? 32 : 4;
     const int S = m->S;  // rows of every product: one per stream
@@ -1125,11 +1328,7 @@ grx_status enqueue_step(grx_whisper *m, hipStream_t stream) {
         a.hist_stream = hp.n_text_ctx;
         return a;
     };
-    // Several streams: the product's prologue builds each stream's row with
-    // one wave per row (rows up to 1280 values); wider rows are LayerNorm'd
-    // and rounded once by a row kernel and read pre-rounded
-    // (GRX_FUSE_LN=0 takes that route for every width).
-    const bool sep = S > 1 && (st > 1280 || tuned_off(GRX_TUNE_FUSE_LN));
+    const bool sep = sep_ln(m);
     auto ln_rows = [&](const float *w, const float *b, GemvArgs &a) {
         a.xq = m->ln_q;
         a.xs = m->ln_s;
@@ -1190,21 +1389,13 @@ grx_status enqueue_step(grx_whisper *m, hipStream_t stream) {
                 pro = GRX_PRO_PREQ;
                 a.xq = m->ln_q;
                 a.xs = m->ln_s;
-                s = li == 0 ? grx_embed_ln_quant_rows(stream, m->tok, m->pos, m->tok_emb, m->dec_pos, m->x, S,
+                s = li == 0 ? grx_embed_ln_quant_rows(stream, m->tok, m->pos, m->tok_emb, m->dec_pos, m->x, S, 1,
                                                       L.attn_ln_w, L.attn_ln_b, m->ln_q, m->ln_s)
                             : grx_ln_quant_rows(stream, m->x, st, S, st, L.attn_ln_w, L.attn_ln_b, m->ln_q, m->ln_s);
                 if (s != GRX_OK) return s;
             }
             if ((s = grx_gemv_launch(stream, S, pro, GRX_EPI_QKV, a, 0)) != GRX_OK) return s;
-            if (qatt)
-                self_attn_kernel<true><<<dim3(nh, S), kAttnThreads, attn_smem, stream>>>(
-                    m->q, L.self_k, L.self_v, m->pos, st, hd, sc, rc, kv_stream, m->att, m->att_q, m->att_s,
-                    hp.n_text_ctx);
-            else
-                self_attn_kernel<false><<<dim3(nh, S), kAttnThreads, attn_smem, stream>>>(
-                    m->q, L.self_k, L.self_v, m->pos, st, hd, sc, rc, kv_stream, m->att, nullptr, nullptr,
-                    hp.n_text_ctx);
-            GRX_LAUNCHED("self_attn_kernel");
+            if ((s = launch_self_attn(m, stream, L, m->q, 1, m->att, m->att_q, m->att_s)) != GRX_OK) return s;
         }
         auto out_proj = [&](grx_weight *w, const float *b, bool rounded) {  // x += att . W^T + b
             if (S > 1 && w->nb <= 128) {
@@ -1324,32 +1515,7 @@ grx_status enqueue_step(grx_whisper *m, hipStream_t stream) {
             if ((s = grx_gemv_launch(stream, S, GRX_PRO_PREQ, GRX_EPI_RESID, a, 0)) != GRX_OK) return s;
         }
     }
-    {  // LN -> logits = tokEmb . h -> argmax; the last workgroup ends the step
-        GemvArgs a = gemv_args(m->tok_emb);
-        a.cacheable = 0;  // 26.5 MB streamed once per step: non-temporal loads
-        a.x = m->x;
-        a.lda = st;
-        a.ln_w = m->dec_ln_w;
-        a.ln_b = m->dec_ln_b;
-        a.y = m->logits;
-        a.ldc = hp.n_vocab;
-        // per-workgroup argmax keys and a one-workgroup end of step (no
-        // contended atomics); ARGMAX_ATOMIC tuned to 1 takes the atomic form
-        const bool atomic_form = grx_tune(GRX_TUNE_ARGMAX_ATOMIC) == 1;
-        a.amax = m->amax;
-        if (atomic_form)
-            a.counter = m->counter;
-        else
-            a.keys = m->keys;
-        a.tok_w = m->tok;
-        a.pos = m->pos;
-        a.pos_w = m->pos;
-        a.hist = m->hist;
-        if (sep && (s = ln_rows(m->dec_ln_w, m->dec_ln_b, a)) != GRX_OK) return s;
-        if ((s = grx_gemv_launch(stream, S, sep ? GRX_PRO_PREQ : GRX_PRO_LN, GRX_EPI_ARGMAX, a, 0)) != GRX_OK)
-            return s;
-    }
-    return GRX_OK;
+    return enqueue_logits(m, stream);
 }
 
 // One step: the captured graph, or (GRX_NO_GRAPH=1, or capture refused)
@@ -1521,7 +1687,9 @@ extern "C" grx_status grx_whisper_decode(grx_whisper *m, const int32_t *tokens, 
         if (tokens[i] < 0 || tokens[i] >= m->hp.n_vocab)
             return grx_fail(GRX_EINVAL, "grx_whisper_decode: token %d out of the vocabulary", tokens[i]);
     hipStream_t stream = m->ctx->stream;
-    for (int i = 0; i < n; ++i) {
+    const bool rows = n >= kPromptMin && prompt_rows_ok(m);
+    if (rows && (s = run_prompt(m, tokens, n)) != GRX_OK) return s;
+    for (int i = 0; !rows && i < n; ++i) {
         GRX_HIP(hipMemcpyAsync(m->tok, tokens + i, 4, hipMemcpyHostToDevice, stream));
         if ((s = run_step(m)) != GRX_OK) return s;
         m->pos_host++;
@@ -1572,7 +1740,9 @@ extern "C" grx_status grx_whisper_greedy_streams(grx_whisper *m, const int32_t *
     hipStream_t stream = m->ctx->stream;
     // the prompt position by position, every stream's token uploaded first
     std::vector<int32_t> col(S);
-    for (int i = 0; i < n_prompt; ++i) {
+    const bool rows = n_prompt >= kPromptMin && prompt_rows_ok(m);
+    if (rows && (s = run_prompt(m, prompts, n_prompt)) != GRX_OK) return s;
+    for (int i = 0; !rows && i < n_prompt; ++i) {
         for (int k = 0; k < S; ++k) col[k] = prompts[(size_t)k * n_prompt + i];
         GRX_HIP(hipMemcpyAsync(m->tok, col.data(), (size_t)S * 4, hipMemcpyHostToDevice, stream));
         if ((s = run_step(m)) != GRX_OK) return s;

@@ -119,6 +119,47 @@ def test_greedy_tokens_identical_and_eager_equals_graph(kern, orc):
     assert list(dec.greedy([1, 2, 3, 4], 40)) == list(want)
 
 
+@pytest.mark.parametrize("nctx", [7, 16, 96, 101, 1500])
+@pytest.mark.parametrize("n", [3, 15, 17, 40])
+def test_prompt_rows_bit_exact(kern, orc, n, nctx):
+    """A prompt decoded as rows of many-row products: its last row's logits,
+    then a second prompt on top and two steps (so every row's keys and
+    values count), bit-identical; audio lengths without and with whole steps
+    of 16, odd ones (values read as single floats), and row groups of 16
+    with and without a remainder."""
+    hp = dict(WHISPER_TINY_TEST, n_audio_ctx=nctx, n_text_ctx=96)
+    ref, dec = _pair(orc, hp, seed=n)
+    rng = np.random.default_rng(n)
+    for m in (n, n, 1, 1):
+        toks = rng.integers(0, hp["n_vocab"], m).tolist()
+        lr = ref.decode(toks)
+        lg, nxt = dec.decode(toks)
+        assert _same(lg, lr), f"{m} at {dec.pos}: max |diff| {np.abs(lg - lr).max()}"
+        assert nxt == orc.argmax(lr)
+    assert dec.pos == 2 * n + 2
+
+
+@pytest.mark.parametrize("streams", [1, 8])
+def test_prompt_passes_equal_steps(kern, orc, streams):
+    """A prompt longer than one pass of rows, for one stream and for eight,
+    against the same prompt token by token (PROMPT_ROWS=0)."""
+    from gorelaxor_amd.whisper import WhisperDecoder
+
+    hp = dict(WHISPER_TINY_TEST, n_text_ctx=320, n_state=320, n_head=5)
+    t = whisper_model(hp, seed=4)
+    prompts = np.random.default_rng(4).integers(0, hp["n_vocab"], (streams, 290 if streams == 1 else 37)).astype(np.int32)
+    out = []
+    for rows in (1, 0):
+        with kern.tuned(PROMPT_ROWS=rows):
+            dec = WhisperDecoder(hp, t, streams=streams)
+            for k in range(streams):
+                dec.set_encoder_output_stream(k, encoder_output(hp, seed=40 + k))
+            first = dec.greedy_streams(prompts, 5) if streams > 1 else dec.greedy(prompts[0].tolist(), 5)
+            out.append((np.asarray(first), np.stack([dec.logits(k) for k in range(streams)])))
+    assert np.array_equal(out[0][0], out[1][0])
+    assert _same(out[0][1], out[1][1])
+
+
 def test_context_limit_and_errors(kern, orc):
     from gorelaxor_amd import GrxError
     from gorelaxor_amd.whisper import WhisperDecoder
