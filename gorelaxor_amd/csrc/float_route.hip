@@ -26,106 +26,202 @@ namespace {
 // gemm.go:116-185) applied to each of B groups of `per` rows: with more than
 // 16 rows, the rows in whole groups of six take k6x16 (kernels_amd64.s:5-88):
 // from the bias (0 without one), each chunk of 256 k's fma chain (from zero)
-// is added in.  This kernel computes that form for every row, 64 rows x 64
-// columns per workgroup, 4 x 4 outputs per thread, 32 k's of x and w staged
-// in LDS per pass (k's past the end staged as zeros: fma(0, 0, acc) leaves a
-// chain that started at +0 unchanged); the rows the reference sends to
-// gemvRows are rewritten afterwards by f32_rows_gemv_kernel.
-constexpr int kPwT = 64, kPwK = 32;
-__global__ __launch_bounds__(256) void f32_rows_k6x16_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                                             const float *__restrict__ bias, float *__restrict__ y,
-                                                             int rows, int n, int k) {
-    __shared__ __align__(16) float as[kPwK][kPwT + 4];
-    __shared__ __align__(16) float ws[kPwK][kPwT + 4];
-    const int tid = threadIdx.x, tr = tid / 16, tc = tid % 16;
-    const int r0 = blockIdx.y * kPwT, c0 = blockIdx.x * kPwT;
-    float acc[4][4], out[4][4];
+// is added in.  This kernel computes that form for every row; the rows the
+// reference sends to gemvRows are rewritten afterwards by
+// f32_rows_gemv_kernel.
+//
+// On the float32 matrix cores: v_mfma_f32_16x16x4_f32 adds its four products
+// to the accumulator one after another in k order with one rounding each,
+// which is four steps of the chain (checked bit for bit against fmaf chains,
+// with subnormal sums, signed zeros, infinities and NaN).  A workgroup of
+// WR x WC waves computes 16 WR RF x 16 WC CF outputs, KC k's a pass through
+// LDS, double-buffered.  Within each 16 k's LDS holds k = 4s + l at place
+// 4l + s, so that lane (i, l)'s operands of four instructions are one 16-byte
+// read; rows are KC + 4 floats apart (those reads of 16 rows fall in distinct
+// banks).  A k past the end is staged as the product of -0 and 0, which
+// leaves every sum as it is.
+//
+// Bound by the matrix cores' float32 rate for many rows (128,512 x 256 x 256:
+// 321 us on a VALU tile, 189 us here, 89 TFLOP/s), by the passes' memory latency for few, which is why those take
+// longer passes and smaller tiles (512 x 256 x 256:
+// 63 -> 6.3 us).
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+template <int WR, int WC, int RF, int CF, int KC>
+struct RowsTile {
+    static constexpr int TM = 16 * WR * RF, TN = 16 * WC * CF, NT = 64 * WR * WC, LD = KC + 4;
+    static constexpr int kBuf = (TM + TN) * LD;
+    static constexpr size_t lds = 2 * kBuf * sizeof(float);
+};
+
+template <int WR, int WC, int RF, int CF, int KC, bool VEC>
+__global__ __launch_bounds__(64 * WR *WC) void f32_rows_mfma_kernel(const float *__restrict__ x,
+                                                                    const float *__restrict__ w,
+                                                                    const float *__restrict__ bias,
+                                                                    float *__restrict__ y, int rows, int n, int k) {
+    using T = RowsTile<WR, WC, RF, CF, KC>;
+    static_assert(256 % KC == 0 && KC % 16 == 0, "chunks of 256 k's end with a pass");
+    constexpr int P = KC / 4;                                    // 16-byte pieces of a row and pass
+    constexpr int NP = ((T::TM + T::TN) * P + T::NT - 1) / T::NT;  // pieces a thread
+    extern __shared__ __align__(16) float st[];
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wave / WC, wc = wave % WC;
+    const int r0 = blockIdx.y * T::TM, c0 = blockIdx.x * T::TN;
+    float4 pre[NP];
+    auto gload = [&](int k0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int col = c0 + tc * 4 + j;
+        for (int u = 0; u < NP; ++u) {
+            const int e = tid + u * T::NT, row = e / P, kk = k0 + 4 * (e % P);
+            const bool isx = row < T::TM;
+            const float pad = isx ? -0.0f : 0.0f;
+            float4 v = make_float4(pad, pad, pad, pad);
+            const int g = isx ? r0 + row : c0 + row - T::TM;
+            if (row < T::TM + T::TN && g < (isx ? rows : n)) {
+                const float *p = (isx ? x : w) + (size_t)g * k + kk;
+                if constexpr (VEC) {  // k % 4 == 0, 16-byte aligned rows
+                    if (kk < k) v = *reinterpret_cast<const float4 *>(p);
+                } else {
+                    if (kk < k) v.x = p[0];
+                    if (kk + 1 < k) v.y = p[1];
+                    if (kk + 2 < k) v.z = p[2];
+                    if (kk + 3 < k) v.w = p[3];
+                }
+            }
+            pre[u] = v;
+        }
+    };
+    auto lstore = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < NP; ++u) {
+            const int e = tid + u * T::NT, row = e / P, pc = e % P;
+            if (row >= T::TM + T::TN) break;
+            float *d = st + buf * T::kBuf + row * T::LD + 16 * (pc >> 2) + (pc & 3);
+            d[0] = pre[u].x;
+            d[4] = pre[u].y;
+            d[8] = pre[u].z;
+            d[12] = pre[u].w;
+        }
+    };
+    v4f acc[RF][CF], out[RF][CF];
+#pragma unroll
+    for (int j = 0; j < CF; ++j) {
+        const int col = c0 + 16 * (wc * CF + j) + li;
         const float bj = (bias != nullptr && col < n) ? bias[col] : 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            out[i][j] = bj;
-            acc[i][j] = 0.f;
+        for (int i = 0; i < RF; ++i) {
+            out[i][j] = v4f{bj, bj, bj, bj};
+            acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
         }
     }
-    for (int k0 = 0; k0 < k; k0 += kPwK) {
-        for (int e = tid; e < kPwT * kPwK; e += 256) {
-            const int rr = e / kPwK, kk = e % kPwK, gr = r0 + rr, gc = c0 + rr;
-            const bool kin = k0 + kk < k;
-            as[kk][rr] = (gr < rows && kin) ? x[(size_t)gr * k + k0 + kk] : 0.f;
-            ws[kk][rr] = (gc < n && kin) ? w[(size_t)gc * k + k0 + kk] : 0.f;
+    gload(0);
+    lstore(0);
+    __syncthreads();
+    int buf = 0;
+    for (int k0 = 0; k0 < k; k0 += KC) {
+        const bool more = k0 + KC < k;
+        if (more) gload(k0 + KC);
+        const float *a0 = st + buf * T::kBuf + (wr * RF * 16 + li) * T::LD + 4 * lk;
+        const float *b0 = st + buf * T::kBuf + (T::TM + wc * CF * 16 + li) * T::LD + 4 * lk;
+#pragma unroll
+        for (int g = 0; g < KC / 16; ++g) {
+            float4 a[RF], b[CF];
+#pragma unroll
+            for (int i = 0; i < RF; ++i) a[i] = *reinterpret_cast<const float4 *>(a0 + 16 * i * T::LD + 16 * g);
+#pragma unroll
+            for (int j = 0; j < CF; ++j) b[j] = *reinterpret_cast<const float4 *>(b0 + 16 * j * T::LD + 16 * g);
+            auto step = [&](auto get) {
+#pragma unroll
+                for (int i = 0; i < RF; ++i)
+#pragma unroll
+                    for (int j = 0; j < CF; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(get(a[i]), get(b[j]), acc[i][j], 0, 0, 0);
+            };
+            step([](const float4 &v) { return v.x; });
+            step([](const float4 &v) { return v.y; });
+            step([](const float4 &v) { return v.z; });
+            step([](const float4 &v) { return v.w; });
         }
-        __syncthreads();
-#pragma unroll 8
-        for (int kk = 0; kk < kPwK; ++kk) {
-            const float4 a = *reinterpret_cast<const float4 *>(&as[kk][tr * 4]);
-            const float4 b = *reinterpret_cast<const float4 *>(&ws[kk][tc * 4]);
-            const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+        if ((k0 + KC) % 256 == 0 || !more) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < RF; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __fmaf_rn(av[i], bv[j], acc[i][j]);
+                for (int j = 0; j < CF; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        out[i][j][r] = __fadd_rn(acc[i][j][r], out[i][j][r]);
+                        acc[i][j][r] = 0.f;
+                    }
         }
-        __syncthreads();
-        if ((k0 + kPwK) % 256 == 0 || k0 + kPwK >= k) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    out[i][j] = __fadd_rn(acc[i][j], out[i][j]);
-                    acc[i][j] = 0.f;
-                }
+        if (more) {
+            lstore(buf ^ 1);  // the other buffer: its readers passed the last barrier
+            __syncthreads();
+            buf ^= 1;
         }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = r0 + tr * 4 + i;
-        if (row >= rows) continue;
+    for (int i = 0; i < RF; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int col = c0 + tc * 4 + j;
-            if (col < n) y[(size_t)row * n + col] = out[i][j];
+        for (int j = 0; j < CF; ++j) {
+            const int col = c0 + 16 * (wc * CF + j) + li;
+            if (col >= n) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = r0 + 16 * (wr * RF + i) + 4 * lk + r;
+                if (row < rows) y[(size_t)row * n + col] = out[i][j][r];
+            }
         }
-    }
 }
 
-// The k6x16 form of the rows below lo of each group, one thread per output
-// (for narrow outputs, where the 64 x 64 tiles would idle): from the bias,
-// each chunk of 256 k's fma chain added in.
-__global__ void f32_rows_k6x16_one_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                          const float *__restrict__ bias, float *__restrict__ y, int B, int per,
-                                          int lo, int n, int k) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)B * lo * n) return;
-    const int j = (int)(i % n);
-    const size_t rr = i / n, row = rr / lo * per + rr % lo;
-    const float *a = x + row * k, *b = w + (size_t)j * k;
-    float c = bias != nullptr ? bias[j] : 0.f;
-    for (int k0 = 0; k0 < k; k0 += 256) {
-        const int kn = min(256, k - k0);
-        float acc = 0.f;
-#pragma unroll 8
-        for (int kk = 0; kk < kn; ++kk) acc = __fmaf_rn(a[k0 + kk], b[k0 + kk], acc);
-        c = __fadd_rn(acc, c);
+template <int WR, int WC, int RF, int CF, int KC>
+hipError_t launch_rows(hipStream_t st, const float *x, const float *w, const float *bias, float *y, int rows, int n,
+                       int k) {
+    using T = RowsTile<WR, WC, RF, CF, KC>;
+    const bool vec = k % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
+    auto kern = vec ? f32_rows_mfma_kernel<WR, WC, RF, CF, KC, true> : f32_rows_mfma_kernel<WR, WC, RF, CF, KC, false>;
+    if constexpr (T::lds > 64 * 1024) {
+        static const hipError_t ok = [] {
+            const hipError_t e = hipFuncSetAttribute((const void *)f32_rows_mfma_kernel<WR, WC, RF, CF, KC, true>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::lds);
+            return e != hipSuccess ? e
+                                   : hipFuncSetAttribute((const void *)f32_rows_mfma_kernel<WR, WC, RF, CF, KC, false>,
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::lds);
+        }();
+        if (ok != hipSuccess) return ok;
     }
-    y[row * n + j] = c;
+    kern<<<dim3((n + T::TN - 1) / T::TN, (rows + T::TM - 1) / T::TM), T::NT, T::lds, st>>>(x, w, bias, y, rows, n, k);
+    return hipGetLastError();
 }
 
 // The rows of each group that ws.matmul sends to gemvRows (gemm.go:
 // 182-184, 195-259): rows lo..per-1 of every group (all of them when
 // per <= 16): dotF32x4 for whole groups of four columns, dotF32Go for the
-// rest, then the bias added (none without one).  One thread per output.
-__global__ void f32_rows_gemv_kernel(const float *__restrict__ x, const float *__restrict__ w,
-                                     const float *__restrict__ bias, float *__restrict__ y, int B, int per, int lo,
-                                     int n, int k) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x, tail = (size_t)(per - lo);
+// rest, then the bias added (none without one).  Sixteen lanes per output,
+// lane c running dot4f32avx's chain c (5 us at 2 rows x 256 x 256,
+// 12 with one thread per output); the Go forms are lane 0's.
+__global__ __launch_bounds__(256) void f32_rows_gemv_kernel(const float *__restrict__ x, const float *__restrict__ w,
+                                                            const float *__restrict__ bias, float *__restrict__ y,
+                                                            int B, int per, int lo, int n, int k) {
+    const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4, tail = (size_t)(per - lo);
+    const int c = threadIdx.x & 15;
     if (i >= (size_t)B * tail * n) return;
     const int j = (int)(i % n);
     const size_t rr = i / n, row = rr / tail * per + lo + rr % tail;
     const float *xr = x + row * k, *wj = w + (size_t)j * k;
-    const float o = j < (n & ~3) ? dot_x4_s(xr, wj, 1, k) : dot_go_s(xr, wj, 1, k);
+    const bool avx = j < (n & ~3);
+    const int kk = avx ? k & ~15 : 0;
+    float acc = 0.f;
+#pragma unroll 8
+    for (int t = c; t < kk; t += 16) acc = __fmaf_rn(xr[t], wj[t], acc);
+    // S_l = A_l + B_l (chains l and 8 + l), h_l = S_l + S_{l+4}, (h0 + h1) + (h2 + h3)
+    float o = __fadd_rn(acc, __shfl_xor(acc, 8, 16));
+    o = __fadd_rn(o, __shfl_xor(o, 4, 16));
+    o = __fadd_rn(o, __shfl_xor(o, 1, 16));
+    o = __fadd_rn(o, __shfl_xor(o, 2, 16));
+    if (c != 0) return;
+    if (kk < k) {
+        const float g = dot_go(xr + kk, wj + kk, k - kk);
+        o = avx ? __fadd_rn(kk > 0 ? o : 0.f, g) : g;
+    }
     y[row * n + j] = bias != nullptr ? __fadd_rn(o, bias[j]) : o;
 }
 
@@ -292,18 +388,18 @@ grx_status grx_float_rows_f32(hipStream_t st, const float *x, const float *w, co
                               int per, int n, int k) {
     const int rows = B * per, lo = per > 16 ? per / 6 * 6 : 0;
     if (rows == 0 || n == 0) return GRX_OK;
-    if (lo > 0 && n < kPwT) {  // narrow outputs: a thread per output
-        const size_t cnt = (size_t)B * lo * n;
-        f32_rows_k6x16_one_kernel<<<(unsigned)((cnt + 255) / 256), 256, 0, st>>>(x, w, bias, y, B, per, lo, n, k);
-        GRX_LAUNCHED("f32_rows_k6x16_one_kernel");
-    } else if (lo > 0) {
-        f32_rows_k6x16_kernel<<<dim3((n + kPwT - 1) / kPwT, (rows + kPwT - 1) / kPwT), 256, 0, st>>>(x, w, bias, y,
-                                                                                                     rows, n, k);
-        GRX_LAUNCHED("f32_rows_k6x16_kernel");
+    if (lo > 0) {
+        // 16 columns a workgroup for narrow outputs; 64 x 64 tiles once they
+        // give two workgroups a CU, 32 x 32 (four times as many) below that
+        const long tiles = (long)grx_ceil_div(rows, 64) * grx_ceil_div(n, 64);
+        const hipError_t e = n <= 32         ? launch_rows<4, 1, 1, 1, 64>(st, x, w, bias, y, rows, n, k)
+                             : tiles >= 512 ? launch_rows<2, 2, 2, 2, 32>(st, x, w, bias, y, rows, n, k)
+                                            : launch_rows<2, 2, 1, 1, 128>(st, x, w, bias, y, rows, n, k);
+        if (e != hipSuccess) return grx_hip_fail(e, "f32_rows_mfma_kernel");
     }
     const size_t tail = (size_t)B * (per - lo) * n;
     if (tail > 0) {
-        f32_rows_gemv_kernel<<<(unsigned)((tail + 255) / 256), 256, 0, st>>>(x, w, bias, y, B, per, lo, n, k);
+        f32_rows_gemv_kernel<<<(unsigned)((tail + 15) / 16), 256, 0, st>>>(x, w, bias, y, B, per, lo, n, k);
         GRX_LAUNCHED("f32_rows_gemv_kernel");
     }
     return GRX_OK;

@@ -38,6 +38,22 @@ def test_tiny_streamed_bit_exact(kern, orc, q8):
     dec.close()
 
 
+@pytest.mark.parametrize("nf", [6, 22, 34])
+def test_float_rows_odd_widths_bit_exact(kern, orc, nf):
+    """float32 convolutions whose row lengths are no multiple of 4 (rows read
+    as single floats) or of 16, past 256 (two chunks, the second partial),
+    and whose output counts leave partial tiles of 16 and of 32 columns."""
+    hp = dict(MIMI_TINY, nf=nf)
+    t = mimi_model(hp, seed=31, q8=False)
+    ref, dec = _pair(orc, hp, t)
+    lat = mimi_latents(hp, 8, seed=32)
+    for i in range(0, 8, 4):
+        want = ref.decode(lat[i:i + 4])
+        got = dec.decode(lat[i:i + 4])
+        assert _same(got, want), f"latents {i}: max |diff| {np.abs(got - want).max()}"
+    dec.close()
+
+
 @pytest.mark.parametrize("mx", [-1, 0])
 @pytest.mark.parametrize("per_call", [2, 3, 4])
 def test_tiny_several_latents_per_call(kern, orc, per_call, mx):
