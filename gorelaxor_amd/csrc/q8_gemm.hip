@@ -29,6 +29,8 @@
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 // The epilogues that round their activation to Q8_0: whole 32-row blocks.
 constexpr bool epi_rounds(int epi) { return epi == GRX_GEMM_SILU_Q || epi == GRX_GEMM_GELU_Q; }
@@ -866,19 +868,48 @@ gemm_q8_kss_kernel(
     }
 }
 
-// The product for many activation rows: a workgroup of eight waves (2 x 4)
-// computes 64 activation rows x 128 weight rows, each wave 32 x 32 (2 x 2
-// MFMA tiles).  kLdsCB blocks at a time of the rounded activations, the two
-// weight tiles, their scales and the activation scales are copied to LDS
-// with 16-byte loads, double-buffered (the next blocks' loads are in flight
-// while the current ones fold), so each activation row and weight row is
-// read from L2 once per workgroup instead of once per wave.  Per output the
-// fold is the same: c = fma(f32(s_b) * dw_b, da_b, c), blocks in order.
-constexpr int kLdsCB = 4;
-constexpr int kLdsThreads = 512;
+// A raw buffer resource over the bytes at p (reads past them give zeros).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p, size_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)(bytes < 0x7fffffff ? bytes : 0x7fffffff),
+                                             0x00020000);
+}
 
-template <int EPI>
-__global__ __launch_bounds__(kLdsThreads) void gemm_q8_lds_kernel(const int8_t *__restrict__ qs,
+// The product for many activation rows: a workgroup of WM x WN waves computes
+// 16 FR WM activation rows x 16 FC WN weight rows, each wave FR x FC MFMA
+// tiles.  CB blocks at a time of the rounded activations, the weights and
+// both scales are copied to LDS with 16-byte loads, double-buffered (the next
+// blocks' loads are in flight while the current ones fold), so each
+// activation row and weight row is read from L2 once per workgroup instead
+// of once per wave.
+//
+// Bound by the fold, c = fma(f32(s_b) * dw_b, da_b, c) per output and block
+// in order, on the vector units.  Its convert and multiply are one fma here:
+// the MFMA adds the int32 sum s to the bits of M = 1.5 * 2^23, which reads as
+// the float M + s exactly (|s| <= 2^19), and fma(M + s, dw, -M dw) rounds
+// s dw once: M dw is exact (dw has float16's 11 significant bits, M has two),
+// so the bits are the product's.  Two cases differ: an infinite dw (NaN
+// instead of an infinity) and the sign of a zero product of a zero or
+// negative dw.  A workgroup that meets such a scale takes the convert and
+// the multiply from there on.
+constexpr uint32_t kFoldMagic = 0x4B400000u;  // the bits of M
+constexpr float kFoldM = 12582912.0f;
+
+template <int WM, int WN, int FR, int FC, int CB>
+struct LdsTile {
+    static constexpr int TM = 16 * FR * WM, TN = 16 * FC * WN, NT = 64 * WM * WN;
+    // per buffer: A [TM rows][CB][32] bytes, rows kAr apart (16 bytes of
+    // padding: a fragment's 8-byte reads of 16 rows and a row's 16-byte
+    // stores fall in distinct banks), B [CB][2 halves][TN][16], weight scales
+    // [CB][TN] f32, activation scales [CB][TM] f32
+    static constexpr int kAr = CB * 32 + 16;
+    static constexpr int kA = TM * kAr, kB = CB * 32 * TN, kD = CB * TN * 4, kS = CB * TM * 4;
+    static constexpr int kBuf = kA + kB + kD + kS;
+    static_assert(64 % TN == 0 || TN % 64 == 0, "weight tiles of 64 rows");
+    static_assert(2 * kBuf <= 64 * 1024, "static LDS");
+};
+
+template <int EPI, int WM, int WN, int FR, int FC, int CB>
+__global__ __launch_bounds__(64 * WM *WN, FR *FC == 4 ? 4 : 2) void gemm_q8_lds_kernel(const int8_t *__restrict__ qs,
                                                                   const uint16_t *__restrict__ ds, int rows, int nb,
                                                                   int tiles, const int8_t *__restrict__ xq,
                                                                   const float *__restrict__ xs, int m,
@@ -886,168 +917,242 @@ __global__ __launch_bounds__(kLdsThreads) void gemm_q8_lds_kernel(const int8_t *
                                                                   float *__restrict__ y, int ldc, float scale,
                                                                   int8_t *__restrict__ yq, float *__restrict__ ys,
                                                                   const KsFuse fz) {
-    // LDS per buffer: A [64 rows][CB][32] bytes, rows kAr apart (16 bytes of
-    // padding: a fragment's 8-byte reads of 16 rows and a row's 16-byte
-    // stores fall in distinct banks), B [CB][2 tiles][2 halves][64][16],
-    // weight scales [CB][128] u16, activation scales [CB][64] f32
-    constexpr int kAr = kLdsCB * 32 + 16;
-    constexpr int kA = 64 * kAr, kB = kLdsCB * 2 * 2048, kD = kLdsCB * 128 * 2, kS = kLdsCB * 64 * 4;
-    constexpr int kBuf = kA + kB + kD + kS;
-    __shared__ __align__(16) uint8_t lds[2 * kBuf];
+    using T = LdsTile<WM, WN, FR, FC, CB>;
+    constexpr int NT = T::NT;
+    static_assert(FC == 2 || (!epi_rounds(EPI) && EPI != GRX_GEMM_GLU), "whole 32-column groups");
+    __shared__ __align__(16) uint8_t lds[2 * T::kBuf];
+    __shared__ int odd;  // a scale that is not positive and finite has come
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 2, wn = wave & 3;             // wave rows 32*wm.., columns 32*wn..
-    const int mb = blockIdx.x * 64, t0 = blockIdx.y * 2;  // activation rows mb.., weight tiles t0, t0+1
+    const int wm = wave / WN, wn = wave % WN;  // wave rows 16 FR wm.., columns 16 FC wn..
+    // Workgroup i runs on XCD i % 8: each XCD takes one run of the tiles,
+    // row groups of a column group together, so that a column group's
+    // weights come into one L2
+    const int nrg = (m + T::TM - 1) / T::TM, total = gridDim.x;
+    const int xcd = blockIdx.x & 7, id = xcd * (total >> 3) + min(xcd, total & 7) + (blockIdx.x >> 3);
+    const int mb = (id % nrg) * T::TM, nc = (id / nrg) * T::TN;  // activation rows mb.., weight rows nc..
     const int K = nb * GRX_QK;
     const int li = lane & 15, lk = lane >> 4;
+    if (tid == 0) odd = 0;
 
-    // ---- the copy of blocks [b0, b0+CB) into registers, then LDS
-    // A: 64 rows x CB*32 bytes = 64 x (2*CB) 16-byte pieces (one per thread for CB 4)
-    // B: 2 tiles x CB x 2048 bytes = 2*CB*128 pieces (two per thread)
-    // dw: 2 tiles x CB x 128 bytes = 2*CB*8 pieces; da: 64 rows x CB floats (one piece per row)
-    constexpr int kApc = 64 * 2 * kLdsCB, kBpc = 2 * kLdsCB * 128, kDpc = 2 * kLdsCB * 8;
-    static_assert(kApc == kLdsThreads && kBpc == 2 * kLdsThreads, "copy split assumes CB 4 and 512 threads");
-    uint4 ra, rb[2], rd;
-    float4 rs;
-    auto gload = [&](int b0) {
-        {
-            const int row = tid / (2 * kLdsCB), piece = tid % (2 * kLdsCB);
-            const int gr = mb + row, bb = b0 + piece / 2;
-            ra = (gr < m && bb < nb) ? *reinterpret_cast<const uint4 *>(xq + (size_t)gr * K + (size_t)bb * 32 + 16 * (piece & 1))
-                                     : make_uint4(0, 0, 0, 0);
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int pc = tid + h * kLdsThreads;
-            const int t = pc / (kLdsCB * 128), rem = pc % (kLdsCB * 128), u = rem / 128, off = rem % 128;
-            const int tile = t0 + t, bb = b0 + u;
-            rb[h] = (tile < tiles && bb < nb)
-                        ? *reinterpret_cast<const uint4 *>(qs + ((size_t)tile * nb + bb) * 2048 + 16 * off)
-                        : make_uint4(0, 0, 0, 0);
-        }
-        if (tid < kDpc) {
-            const int t = tid / (kLdsCB * 8), rem = tid % (kLdsCB * 8), u = rem / 8, off = rem % 8;
-            const int tile = t0 + t, bb = b0 + u;
-            rd = (tile < tiles && bb < nb)
-                     ? *reinterpret_cast<const uint4 *>(ds + ((size_t)tile * nb + bb) * 64 + 8 * off)
-                     : make_uint4(0, 0, 0, 0);
-        }
-        if (tid >= kDpc && tid < kDpc + 64) {
-            const int row = tid - kDpc, gr = mb + row;
-#pragma unroll
-            for (int u = 0; u < kLdsCB; ++u) {
-                const float v = (gr < m && b0 + u < nb) ? xs[(size_t)gr * nb + b0 + u] : 0.0f;
-                if (u == 0) rs.x = v;
-                if (u == 1) rs.y = v;
-                if (u == 2) rs.z = v;
-                if (u == 3) rs.w = v;
-            }
-        }
+    // ---- the copy of blocks [b0, b0+CB) into registers, then LDS, in pieces
+    // of 16 bytes and single scales.  Nothing branches: a load whose result
+    // one side of a branch leaves unused holds up the loads after it.
+    // Threads past the pieces repeat the first ones.
+    constexpr int kApc = T::TM * 2 * CB, kBpc = T::TN * 2 * CB, kDpc = T::TN * CB, kSpc = T::TM * CB;
+    constexpr int NA = (kApc + NT - 1) / NT, NB = (kBpc + NT - 1) / NT;
+    constexpr int ND = (kDpc + NT - 1) / NT, NS = (kSpc + NT - 1) / NT;
+    struct Set {
+        v4u a[NA], b[NB];
+        uint16_t d[ND];
+        float s[NS];
     };
-    auto lstore = [&](int buf) {
-        uint8_t *base = lds + buf * kBuf;
-        {
-            const int row = tid / (2 * kLdsCB), piece = tid % (2 * kLdsCB);
-            *reinterpret_cast<uint4 *>(base + row * kAr + 16 * piece) = ra;
+    // through buffer resources that start at the workgroup's first row and
+    // weight tile (the scalar offset is no part of their range check, so the
+    // stage is added to the lane's): rows and blocks past the operands read
+    // as zeros, which nothing uses
+    const int t0 = nc >> 6;
+    const auto rxq = buf_rsrc(xq + (size_t)mb * K, (size_t)(m - mb) * K);
+    const auto rxs = buf_rsrc(xs + (size_t)mb * nb, (size_t)(m - mb) * nb * 4);
+    const auto rqs = buf_rsrc(qs + (size_t)t0 * nb * 2048, (size_t)(tiles - t0) * nb * 2048);
+    const auto rds = buf_rsrc(ds + (size_t)t0 * nb * 64, (size_t)(tiles - t0) * nb * 128);
+    int oa[NA], ob[NB], od[ND], os[NS];
+#pragma unroll
+    for (int h = 0; h < NA; ++h) {
+        const int pc = (tid + h * NT) % kApc;
+        oa[h] = pc / (2 * CB) * K + 16 * (pc % (2 * CB));
+    }
+#pragma unroll
+    for (int h = 0; h < NB; ++h) {
+        const int pc = (tid + h * NT) % kBpc, col = (nc & 63) + pc % T::TN, half = pc / T::TN;  // half 2u + h of block u
+        ob[h] = ((col >> 6) * nb + (half >> 1)) * 2048 + 1024 * (half & 1) + 16 * (col & 63);
+    }
+#pragma unroll
+    for (int h = 0; h < ND; ++h) {
+        const int pc = (tid + h * NT) % kDpc, col = (nc & 63) + pc % T::TN;
+        od[h] = ((col >> 6) * nb + pc / T::TN) * 128 + 2 * (col & 63);
+    }
+#pragma unroll
+    for (int h = 0; h < NS; ++h) {
+        const int pc = (tid + h * NT) % kSpc;
+        os[h] = 4 * (pc / CB * nb + pc % CB);
+    }
+    auto gload = [&](Set &S, int b0) {
+#pragma unroll
+        for (int h = 0; h < NA; ++h) S.a[h] = __builtin_amdgcn_raw_buffer_load_b128(rxq, oa[h] + b0 * 32, 0, 0);
+#pragma unroll
+        for (int h = 0; h < NB; ++h) S.b[h] = __builtin_amdgcn_raw_buffer_load_b128(rqs, ob[h] + b0 * 2048, 0, 0);
+#pragma unroll
+        for (int h = 0; h < ND; ++h) S.d[h] = __builtin_amdgcn_raw_buffer_load_b16(rds, od[h] + b0 * 128, 0, 0);
+#pragma unroll
+        for (int h = 0; h < NS; ++h)
+            S.s[h] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rxs, os[h] + b0 * 4, 0, 0));
+    };
+    auto lstore = [&](const Set &S, int buf) {
+        uint8_t *base = lds + buf * T::kBuf;
+        float *dl = reinterpret_cast<float *>(base + T::kA + T::kB), *sl = dl + CB * T::TN;
+#pragma unroll
+        for (int h = 0; h < NA; ++h) {
+            const int pc = (tid + h * NT) % kApc;
+            *reinterpret_cast<v4u *>(base + (pc / (2 * CB)) * T::kAr + 16 * (pc % (2 * CB))) = S.a[h];
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int pc = tid + h * kLdsThreads;
-            const int t = pc / (kLdsCB * 128), rem = pc % (kLdsCB * 128), u = rem / 128, off = rem % 128;
-            *reinterpret_cast<uint4 *>(base + kA + (u * 2 + t) * 2048 + 16 * off) = rb[h];
+        for (int h = 0; h < NB; ++h)
+            *reinterpret_cast<v4u *>(base + T::kA + 16 * ((tid + h * NT) % kBpc)) = S.b[h];
+        bool bad = false;
+#pragma unroll
+        for (int h = 0; h < ND; ++h) {
+            const int pc = (tid + h * NT) % kDpc;
+            dl[pc] = grx_f16_to_f32(S.d[h]);
+            bad |= S.d[h] - 1u >= 0x7bffu && nc + pc % T::TN < rows;
         }
-        if (tid < kDpc) {
-            const int t = tid / (kLdsCB * 8), rem = tid % (kLdsCB * 8), u = rem / 8, off = rem % 8;
-            *reinterpret_cast<uint4 *>(base + kA + kB + (u * 128 + t * 64) * 2 + 16 * off) = rd;
+#pragma unroll
+        for (int h = 0; h < NS; ++h) {
+            const int pc = (tid + h * NT) % kSpc;
+            sl[(pc % CB) * T::TM + pc / CB] = S.s[h];
         }
-        if (tid >= kDpc && tid < kDpc + 64) {
-            const int row = tid - kDpc;
-            float *sa = reinterpret_cast<float *>(base + kA + kB + kD);
-            sa[0 * 64 + row] = rs.x;
-            sa[1 * 64 + row] = rs.y;
-            sa[2 * 64 + row] = rs.z;
-            sa[3 * 64 + row] = rs.w;
-        }
+        if (bad) odd = 1;
     };
 
-    float c[2][2][4];  // [row frag][column frag][r]
+    float c[FR][FC][4];  // [row frag][column frag][r]
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-        const int n = t0 * 64 + 32 * wn + 16 * g + li;
+    for (int g = 0; g < FC; ++g) {
+        const int n = nc + 16 * (FC * wn + g) + li;
         const float bv = (bias != nullptr && n < rows) ? bias[n] : 0.0f;
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int f = 0; f < FR; ++f)
 #pragma unroll
             for (int r = 0; r < 4; ++r) c[f][g][r] = bv;
     }
-    const int nsteps = (nb + kLdsCB - 1) / kLdsCB;
-    gload(0);
-    lstore(0);
-    __syncthreads();
-    for (int st = 0; st < nsteps; ++st) {
-        const int cur = st & 1;
-        if (st + 1 < nsteps) gload((st + 1) * kLdsCB);
-        const uint8_t *base = lds + cur * kBuf;
-        const uint16_t *dwl = reinterpret_cast<const uint16_t *>(base + kA + kB);
-        const float *dal = reinterpret_cast<const float *>(base + kA + kB + kD);
-        const int ub = min(kLdsCB, nb - st * kLdsCB);
+    // a block's operands, its products, their fold
+    struct Ops {
+        long a[FR], b[FC];
+        v4f da[FR];
+        float dw[FC];
+    };
+    auto read = [&](const uint8_t *base, int u) {
+        const float *dwl = reinterpret_cast<const float *>(base + T::kA + T::kB) + 16 * FC * wn + li;
+        const float *dal = reinterpret_cast<const float *>(base + T::kA + T::kB + T::kD) + 16 * FR * wm + 4 * lk;
+        const uint8_t *al = base + (16 * FR * wm + li) * T::kAr + 8 * lk;
+        const uint8_t *bl = base + T::kA + (lk >> 1) * T::TN * 16 + (16 * FC * wn + li) * 16 + 8 * (lk & 1);
+        Ops o;
 #pragma unroll
-        for (int u = 0; u < kLdsCB; ++u) {
-            if (u >= ub) break;
-            long av[2], bv[2];
-            float da[2][4], dw[2];
+        for (int f = 0; f < FR; ++f) {
+            o.a[f] = *reinterpret_cast<const long *>(al + 16 * f * T::kAr + u * 32);
+            o.da[f] = *reinterpret_cast<const v4f *>(dal + u * T::TM + 16 * f);
+        }
 #pragma unroll
-            for (int f = 0; f < 2; ++f) {
-                const int row = 32 * wm + 16 * f + li;
-                av[f] = *reinterpret_cast<const long *>(base + row * kAr + u * 32 + 8 * lk);
+        for (int g = 0; g < FC; ++g) {
+            o.b[g] = *reinterpret_cast<const long *>(bl + (2 * u * T::TN + 16 * g) * 16);
+            o.dw[g] = dwl[u * T::TN + 16 * g];
+        }
+        return o;
+    };
+    struct Dots {
+        v4i d[FR][FC];
+    };
+    auto products = [&](const Ops &o, int z0) {
+        const v4i z = {z0, z0, z0, z0};
+        Dots p;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) da[f][r] = dal[u * 64 + 32 * wm + 16 * f + 4 * lk + r];
-            }
+        for (int f = 0; f < FR; ++f)
 #pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                const int col = 32 * wn + 16 * g + li;  // 0..127 across the two tiles
-                const int t = col >> 6, cr = col & 63;
-                bv[g] = *reinterpret_cast<const long *>(base + kA + (u * 2 + t) * 2048 + (lk >> 1) * 1024 + cr * 16 +
-                                                        8 * (lk & 1));
-                dw[g] = grx_f16_to_f32(dwl[u * 128 + col]);
-            }
-            // the block's four products issued together, then their folds:
-            // no fold waits on a product issued just before it
-            v4i d[2][2];
+            for (int g = 0; g < FC; ++g) p.d[f][g] = __builtin_amdgcn_mfma_i32_16x16x32_i8(o.a[f], o.b[g], z, 0, 0, 0);
+        return p;
+    };
+    auto fold = [&](const Ops &o, const Dots &p, auto plain) {
 #pragma unroll
-            for (int f = 0; f < 2; ++f)
+        for (int g = 0; g < FC; ++g) {
+            const float md = __fmul_rn(-kFoldM, o.dw[g]);
 #pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    const v4i z = {0, 0, 0, 0};
-                    d[f][g] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av[f], bv[g], z, 0, 0, 0);
+            for (int f = 0; f < FR; ++f) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int d = p.d[f][g][r];
+                    const float t = decltype(plain)::value ? __fmul_rn((float)d, o.dw[g])
+                                                           : __fmaf_rn(__int_as_float(d), o.dw[g], md);
+                    c[f][g][r] = __fmaf_rn(t, o.da[f][r], c[f][g][r]);
                 }
-#pragma unroll
-            for (int f = 0; f < 2; ++f)
-#pragma unroll
-                for (int g = 0; g < 2; ++g)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        c[f][g][r] = __fmaf_rn(__fmul_rn((float)d[f][g][r], dw[g]), da[f][r], c[f][g][r]);
+            }
         }
-        if (st + 1 < nsteps) {
-            lstore(cur ^ 1);
-            __syncthreads();
+    };
+    auto blocks = [&](int buf, int st) {
+        const uint8_t *base = lds + buf * T::kBuf;
+        const int ub = min(CB, nb - st * CB);
+        const bool slow = __builtin_amdgcn_readfirstlane(odd) != 0;
+        if (!slow && ub == CB) {
+            if constexpr (FR * FC == 4) {
+                // block by block: registers for two workgroups a CU, whose
+                // waves overlap each other's reads, products and folds
+#pragma unroll
+                for (int u = 0; u < CB; ++u) {
+                    const Ops o = read(base, u);
+                    fold(o, products(o, (int)kFoldMagic), std::false_type{});
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else {
+                // a block's products are issued before the fold of the block
+                // before it, its operands read one block earlier still
+                Ops o0 = read(base, 0), o1 = read(base, 1);
+                Dots p = products(o0, (int)kFoldMagic);
+#pragma unroll
+                for (int u = 0; u < CB; ++u) {
+                    Ops o2;
+                    Dots pn;
+                    if (u + 2 < CB) o2 = read(base, u + 2);
+                    if (u + 1 < CB) pn = products(o1, (int)kFoldMagic);
+                    fold(o0, p, std::false_type{});
+                    o0 = o1;
+                    o1 = o2;
+                    p = pn;
+                }
+            }
+        } else {
+#pragma unroll 1
+            for (int u = 0; u < ub; ++u) {
+                const Ops o = read(base, u);
+                fold(o, products(o, 0), std::true_type{});
+            }
         }
+    };
+    const int nsteps = (nb + CB - 1) / CB;
+    Set s0, s1;
+    gload(s0, 0);
+    gload(s1, CB);
+    __syncthreads();  // odd is 0
+    lstore(s0, 0);
+    __syncthreads();
+    int st = 0;
+    for (; st + 2 < nsteps; st += 2) {
+        gload(s0, (st + 2) * CB);
+        blocks(0, st);
+        lstore(s1, 1);
+        __syncthreads();
+        gload(s1, (st + 3) * CB);
+        blocks(1, st + 1);
+        lstore(s0, 0);
+        __syncthreads();
+    }
+    blocks(0, st);
+    if (st + 1 < nsteps) {
+        lstore(s1, 1);
+        __syncthreads();
+        blocks(1, st + 1);
     }
 
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
+    for (int f = 0; f < FR; ++f) {
         int drow[4];
         bool drow_ok[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            drow[r] = mb + 32 * wm + 16 * f + 4 * lk + r;
+            drow[r] = mb + 16 * (FR * wm + f) + 4 * lk + r;
             drow_ok[r] = drow[r] < m;
         }
         if constexpr (epi_rounds(EPI)) {
             // the wave's 32 columns are one Q8_0 block (rows % 32 == 0)
             const int nr = rows / GRX_QK;
-            const int n0 = t0 * 64 + 32 * wn;
+            const int n0 = nc + 32 * wn;
             const bool col_ok = n0 < rows;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -1081,7 +1186,7 @@ __global__ __launch_bounds__(kLdsThreads) void gemm_q8_lds_kernel(const int8_t *
             // the wave's 32 columns are one pair group (grx_glu_row): its
             // 16 a-rows (g = 0) and their b-rows (g = 1) in the same lane,
             // channel n0/2 + li
-            const int n0 = t0 * 64 + 32 * wn;
+            const int n0 = nc + 32 * wn;
             if (n0 < rows) {
                 const int rh = fz.ring.p != nullptr ? ring_head(fz.ring) : 0;
 #pragma unroll
@@ -1097,8 +1202,8 @@ __global__ __launch_bounds__(kLdsThreads) void gemm_q8_lds_kernel(const int8_t *
         } else {
             const int rh = (EPI == GRX_GEMM_STORE && fz.ring.p != nullptr) ? ring_head(fz.ring) : 0;
 #pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                const int n = t0 * 64 + 32 * wn + 16 * g + li;
+            for (int g = 0; g < FC; ++g) {
+                const int n = nc + 16 * (FC * wn + g) + li;
                 if (n >= rows) continue;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
@@ -1334,16 +1439,48 @@ void launch_ks_fused(hipStream_t st, const grx_weight *w, const int8_t *xq, cons
     return launch_ks_fused_pro<EPI, 2>(st, w, xq, xs, m, bias, o, ns, kb);
 }
 
+template <int EPI, int WM, int WN, int FR, int FC, int CB>
+void launch_lds_tile(hipStream_t st, const grx_weight *w, const int8_t *xq, const float *xs, int m, const float *bias,
+                     const GemmOut &o) {
+    using T = LdsTile<WM, WN, FR, FC, CB>;
+    const int groups = grx_ceil_div(m, T::TM) * grx_ceil_div(w->rows, T::TN);
+    gemm_q8_lds_kernel<EPI, WM, WN, FR, FC, CB><<<groups, T::NT, 0, st>>>(
+        w->qs, w->ds, w->rows, w->nb, w->tiles, xq, xs, m, bias, o.y, o.ldc, o.scale, o.yq, o.ys, ks_fuse(o));
+}
+
+template <int EPI>
+void launch_lds(hipStream_t st, const grx_weight *w, const int8_t *xq, const float *xs, int m, const float *bias,
+                const GemmOut &o) {
+    // 64 x 128 tiles from 144 of them on (two in flight a CU fold fastest:
+    // 2016 x 4096 x 1024 44.5 us against 65 in 64 x 32; 160 tiles of 300 x
+    // 4096 x 1024 16.2 against 17.6, 128 of 1000 x 1024 x 1024 16.9 against
+    // 14.4).  Fewer leave CUs idle: 64 x 32 then (300 x 1024 x 4096, 40 wide
+    // tiles, 45 -> 22.8 us), or 32 x 32 where even those are at most 128
+    // (256 x 1024 x 1024 10.3 -> 9.0 us, 15.8 in 64 x 128).  Whole calls with
+    // the rounding launch.
+    if (grx_ceil_div(m, 64) * grx_ceil_div(w->rows, 128) >= 144)
+        launch_lds_tile<EPI, 2, 4, 2, 2, 4>(st, w, xq, xs, m, bias, o);
+    else if (grx_ceil_div(m, 64) * grx_ceil_div(w->rows, 32) > 128)
+        launch_lds_tile<EPI, 4, 1, 1, 2, 8>(st, w, xq, xs, m, bias, o);
+    else if constexpr (epi_rounds(EPI) || EPI == GRX_GEMM_GLU)
+        launch_lds_tile<EPI, 2, 1, 1, 2, 8>(st, w, xq, xs, m, bias, o);
+    else
+        launch_lds_tile<EPI, 2, 2, 1, 1, 8>(st, w, xq, xs, m, bias, o);
+}
+
 // Which kernel a product takes (GEMM_KERNEL forces one; tests force each
 // with it): the one-row GEMV for one row (a conformer's one-row streaming
 // chunk step, a single latent: the same blocks folded in the same order,
 // its weights streamed once, on slices of the weight tiles where those
 // give more workgroups: 1024 x 4096 6.2 us on 128 workgroups of 8 rows
 // against 8.0 K-split; a forced GEMM_KERNEL keeps the matrix cores); the
-// LDS-staged tiles from 256 rows on;
-// below that the K-split tiles with their activations staged through LDS
-// (at 224 rows: 1024 x 4096 17 us against 26 on the whole-K register walk
-// and 50 on the LDS tiles, 4096 x 1024 12 against 19 and 15); without the
+// LDS-staged tiles from 256 rows on, and from 33 where 64 x 32 tiles of the
+// output are 128 or more (calls with the rounding launch: 126 x 4096 x 1024
+// 10.5 us against 12.3 K-split, 126 x 2048 x 1024 8.8 against 9.8, 240 x 1024
+// x 4096 17.6 against 21.0, 48 x 4096 x 1024 8.9 against 9.8; with 64 tiles
+// the K-split wins: 126 x 1024 x 4096 13.8 against 16.4); below that the
+// K-split tiles with their activations staged through LDS (at 224 rows: 1024
+// x 4096 17 us against 26 on the whole-K register walk); without the
 // staging, the K-split tiles up to 128 rows where the register walk has few
 // tiles or a long K (at 126 rows: 4096 x 1024 10.4 us on the register walk
 // against 11.9 K-split; 2048 x 1024 8.1 against 7.3; 1024 x 4096 25 against
@@ -1369,7 +1506,8 @@ RoutePick pick_route(const grx_weight *w, const int8_t *xq, const float *xs, int
     p.sa = grx_tune(GRX_TUNE_GEMM_STAGE_A) != 0 && p.da4 && (pro || ((uintptr_t)xq & 15) == 0);
     const bool ks_ok = pick_ks(m, w->nb, w->rows, o.epi, o.carry != nullptr, p.sa, pro, &p.ns, &p.kb) &&
                        (kind == 2 || (p.sa ? m < 256 : (m <= 128 && (m <= 32 || w->rows <= 2048 || w->nb > 64))));
-    if (kind == 3 || (kind != 1 && kind != 2 && m >= 256)) {
+    const bool lds = m >= 256 || (m > 32 && p.sa && !pro && grx_ceil_div(m, 64) * grx_ceil_div(w->rows, 32) >= 128);
+    if (kind == 3 || (kind != 1 && kind != 2 && lds)) {
         p.r = kRouteLds;
     } else if (kind != 1 && ks_ok) {
         p.r = kRouteKs;
@@ -1449,23 +1587,16 @@ grx_status grx_gemm_q8_launch_ex(hipStream_t st, const grx_weight *w, const int8
         const int pro = o.x == nullptr ? GRX_PRO_PREQ : o.ln_w2 != nullptr ? GRX_PRO_LN2 : GRX_PRO_LN;
         return grx_gemv_launch(st, 1, pro, epi, a, 0);
     }
-    if (p.r == kRouteLds) {  // many rows: the LDS-staged 64 x 128 tiles
-        dim3 g2(grx_ceil_div(m, 64), grx_ceil_div(w->tiles, 2));
-#define GRX_GEMM_LDS(E)                                                                                           \
-    case E:                                                                                                       \
-        gemm_q8_lds_kernel<E><<<g2, kLdsThreads, 0, st>>>(w->qs, w->ds, w->rows, w->nb, w->tiles, xq, xs, m, bias, \
-                                                          o.y, o.ldc, o.scale, o.yq, o.ys, ks_fuse(o));           \
-        break;
+    if (p.r == kRouteLds) {  // many rows: the LDS-staged tiles
         switch (o.epi) {
-            GRX_GEMM_LDS(GRX_GEMM_STORE)
-            GRX_GEMM_LDS(GRX_GEMM_ADD)
-            GRX_GEMM_LDS(GRX_GEMM_AXPY_HALF)
-            GRX_GEMM_LDS(GRX_GEMM_SCALE)
-            GRX_GEMM_LDS(GRX_GEMM_SILU_Q)
-            GRX_GEMM_LDS(GRX_GEMM_GLU)
-            GRX_GEMM_LDS(GRX_GEMM_GELU_Q)
+            case GRX_GEMM_STORE: launch_lds<GRX_GEMM_STORE>(st, w, xq, xs, m, bias, o); break;
+            case GRX_GEMM_ADD: launch_lds<GRX_GEMM_ADD>(st, w, xq, xs, m, bias, o); break;
+            case GRX_GEMM_AXPY_HALF: launch_lds<GRX_GEMM_AXPY_HALF>(st, w, xq, xs, m, bias, o); break;
+            case GRX_GEMM_SCALE: launch_lds<GRX_GEMM_SCALE>(st, w, xq, xs, m, bias, o); break;
+            case GRX_GEMM_SILU_Q: launch_lds<GRX_GEMM_SILU_Q>(st, w, xq, xs, m, bias, o); break;
+            case GRX_GEMM_GLU: launch_lds<GRX_GEMM_GLU>(st, w, xq, xs, m, bias, o); break;
+            case GRX_GEMM_GELU_Q: launch_lds<GRX_GEMM_GELU_Q>(st, w, xq, xs, m, bias, o); break;
         }
-#undef GRX_GEMM_LDS
         GRX_LAUNCHED("gemm_q8_lds_kernel");
         return GRX_OK;
     }

@@ -286,6 +286,45 @@ def test_matmul_lds_tiles_and_register_tiles(kern, orc, kernel):
                 _check_matmul(kern, orc, rng, m, n, 32 * nb, bias=(m % 2 == 1))
 
 
+@pytest.mark.parametrize("m,n", [(65, 9217), (140, 5800), (65, 2081), (97, 2050), (65, 300), (33, 33)])
+def test_matmul_lds_each_tile(kern, orc, m, n):
+    """The LDS-staged product's tiles (64 x 128, 64 x 32, 32 x 32, by the
+    number of tiles), over block counts around one and two copies of blocks:
+    bit-identical to the oracle."""
+    rng = np.random.default_rng(59 + n)
+    with kern.tuned(GEMM_KERNEL=3):
+        for nb in (1, 3, 4, 5, 8, 9, 16, 17, 21):
+            _check_matmul(kern, orc, rng, m, n, 32 * nb, bias=(nb % 2 == 1))
+
+
+@pytest.mark.parametrize("m,n", [(65, 9217), (65, 2081), (65, 300)])
+@pytest.mark.parametrize("scale", [0x0000, 0x8000, 0xA000, 0x7C00, 0xFC00, 0x7E00, 0x0001, 0x7BFF])
+def test_matmul_lds_unusual_scales(kern, m, n, scale):
+    """Blocks whose scale is zero, negative, infinite, not a number, the
+    least or the greatest one, among ordinary ones, and a bias of -0: the
+    LDS-staged product's one-fma scaling gives the bits of the K-split
+    kernel's convert and multiply (a NaN where that has one)."""
+    rng = np.random.default_rng(scale + n)
+    k = 32 * 20
+    w8 = rng.integers(0, 256, (n, k // 32, 34), dtype=np.uint8)
+    w8[:, :, :2] = (rng.random((n, k // 32)) * 0.02 + 1e-4).astype(np.float16).view(np.uint8).reshape(n, -1, 2)
+    w8[:, :, 2:][rng.random((n, k // 32)) < 0.1] = 0
+    odd = rng.random((n, k // 32)) < 0.02
+    odd[n // 2] = True
+    w8[odd, 0], w8[odd, 1] = scale & 255, scale >> 8
+    w = kern.NewQ8(n, k, w8.reshape(-1))
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    bias = np.where(rng.random(n) < 0.5, np.float32(-0.0), rng.standard_normal(n).astype(np.float32))
+    bias[n // 2] = -0.0
+    got, want = np.zeros((m, n), np.float32), np.zeros((m, n), np.float32)
+    for dst, kernel in ((got, 3), (want, 2)):
+        with kern.tuned(GEMM_KERNEL=kernel):
+            kern.MatMul(dst, n, x, k, m, w, bias)
+    nan = np.isnan(want)
+    np.testing.assert_array_equal(np.isnan(got), nan)
+    np.testing.assert_array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+
+
 @pytest.mark.parametrize("m,n,k", [(126, 4096, 1024), (300, 1024, 1024), (1500, 512, 512), (251, 1024, 1024),
                                    (16, 4096, 1024)])
 def test_matmul_many_rows_bit_exact(kern, orc, m, n, k):
