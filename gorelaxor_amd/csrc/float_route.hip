@@ -19,6 +19,7 @@
 // in LDS.
 #include "grx_float.h"
 #include "grx_internal.h"
+#include "grx_ln.h"
 
 namespace {
 
@@ -260,14 +261,31 @@ __device__ __forceinline__ void stage_x(const float *__restrict__ x, int k, floa
     __syncthreads();
 }
 
+// The row in xs normalized and modulated in place (GrxFloatPro).  Every
+// workgroup does it for itself: a launch of its own in front of a 512 x 512
+// product took 4.4 us and its gap for a row of 2 KB.
+__device__ __forceinline__ void float_prologue(const GrxFloatPro &p, float *xs, int k) {
+    __shared__ double red[48];  // ln_block_reduce
+    double mean, inv;
+    ln64_stats(xs, k, p.eps, red, mean, inv);
+    for (int j = threadIdx.x; j < k; j += blockDim.x) {
+        float o = (float)__dmul_rn(__dsub_rn((double)xs[j], mean), inv);
+        if (p.w) o = __fadd_rn(__fmul_rn(o, p.w[j]), p.b[j]);
+        xs[j] = __fadd_rn(__fmul_rn(o, __fadd_rn(1.f, p.scale[j])), p.shift[j]);
+    }
+    __syncthreads();
+}
+
 // Q8_0: the rows of one tile per workgroup (q8_float_row).
+template <bool LN>
 __global__ __launch_bounds__(256) void q8_float_gemv_kernel(const float *__restrict__ x, int k,
                                                             const int8_t *__restrict__ qs,
                                                             const uint16_t *__restrict__ ds, int nb, int n,
                                                             const float *__restrict__ bias, float *__restrict__ y,
-                                                            GrxFloatEpi e) {
+                                                            GrxFloatEpi e, GrxFloatPro p) {
     extern __shared__ __align__(16) float xs[];
     stage_x(x, k, xs);
+    if constexpr (LN) float_prologue(p, xs, k);
     int row;
     bool emit;
     float o = q8_float_row(xs, qs, ds, nb, n, blockIdx.x, row, emit);
@@ -280,12 +298,14 @@ __global__ __launch_bounds__(256) void q8_float_gemv_kernel(const float *__restr
 // A[l] and B[l] (16 values a step), S[l] = A[l]+B[l], and the HSUM is formed
 // across the eight as (h0+h1)+(h2+h3), h_l = S[l]+S[l+4]; thread 0 adds
 // dotF32Go over k past k &^ 15.  Rows past n &^ 3 take dotF32Go in thread 0.
+template <bool LN>
 __global__ __launch_bounds__(256) void f32_gemv_kernel(const float *__restrict__ x, int k,
                                                        const float *__restrict__ w, int n,
                                                        const float *__restrict__ bias, float *__restrict__ y,
-                                                       GrxFloatEpi e) {
+                                                       GrxFloatEpi e, GrxFloatPro p) {
     extern __shared__ __align__(16) float xs[];
     stage_x(x, k, xs);
+    if constexpr (LN) float_prologue(p, xs, k);
     const int row = blockIdx.x * 32 + (threadIdx.x >> 3), l = threadIdx.x & 7;
     const bool live = row < n, avx = row < (n & ~3);
     const float *wr = w + (size_t)row * k;
@@ -318,20 +338,21 @@ constexpr int kMaxK = 32768;
 }  // namespace
 
 grx_status grx_float_gemv_q8(hipStream_t st, const grx_weight *w, const float *x, const float *bias, float *y,
-                             GrxFloatEpi e) {
+                             GrxFloatEpi e, GrxFloatPro p) {
     if (w->cols > kMaxK) return grx_fail(GRX_ESIZE, "float route: %d columns (at most %d)", w->cols, kMaxK);
     if (w->rows == 0) return GRX_OK;
-    q8_float_gemv_kernel<<<w->tiles, 256, (size_t)w->cols * 4, st>>>(x, w->cols, w->qs, w->ds, w->nb, w->rows, bias,
-                                                                      y, e);
+    auto kern = p.scale ? q8_float_gemv_kernel<true> : q8_float_gemv_kernel<false>;
+    kern<<<w->tiles, 256, (size_t)w->cols * 4, st>>>(x, w->cols, w->qs, w->ds, w->nb, w->rows, bias, y, e, p);
     GRX_LAUNCHED("q8_float_gemv_kernel");
     return GRX_OK;
 }
 
 grx_status grx_float_gemv_f32(hipStream_t st, const float *w, int n, int k, const float *x, const float *bias,
-                              float *y, GrxFloatEpi e) {
+                              float *y, GrxFloatEpi e, GrxFloatPro p) {
     if (k > kMaxK) return grx_fail(GRX_ESIZE, "float route: %d columns (at most %d)", k, kMaxK);
     if (n == 0) return GRX_OK;
-    f32_gemv_kernel<<<grx_ceil_div(n, 32), 256, (size_t)k * 4, st>>>(x, k, w, n, bias, y, e);
+    auto kern = p.scale ? f32_gemv_kernel<true> : f32_gemv_kernel<false>;
+    kern<<<grx_ceil_div(n, 32), 256, (size_t)k * 4, st>>>(x, k, w, n, bias, y, e, p);
     GRX_LAUNCHED("f32_gemv_kernel");
     return GRX_OK;
 }

@@ -46,10 +46,16 @@ struct GrxFloatEpi {
     int kind = GRX_FEPI_STORE;
     const float *gate = nullptr;  // GATE: y[row] += gate[row] * (product + bias)
 };
+// With scale set, x is first n = layerNorm(x) (float64 statistics, gain w and
+// bias b when given) * (1 + scale) + shift, formed by every workgroup.
+struct GrxFloatPro {
+    const float *scale = nullptr, *shift = nullptr, *w = nullptr, *b = nullptr;
+    double eps = 0;
+};
 grx_status grx_float_gemv_q8(hipStream_t st, const grx_weight *w, const float *x, const float *bias, float *y,
-                             GrxFloatEpi e = GrxFloatEpi());
+                             GrxFloatEpi e = GrxFloatEpi(), GrxFloatPro p = GrxFloatPro());
 grx_status grx_float_gemv_f32(hipStream_t st, const float *w, int n, int k, const float *x, const float *bias,
-                              float *y, GrxFloatEpi e = GrxFloatEpi());
+                              float *y, GrxFloatEpi e = GrxFloatEpi(), GrxFloatPro p = GrxFloatPro());
 // kern.Linear of a float32 weight [n][k] over B groups of `per` rows (the
 // k6x16 form for rows in whole groups of six when a group has more than 16,
 // gemvRows for the rest); bias nullable.

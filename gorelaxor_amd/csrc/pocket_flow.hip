@@ -38,8 +38,7 @@ __global__ void flow_prep_kernel(const int *__restrict__ frame, const float *__r
 }
 
 // sy = kern.SiLU(y + tc) over dim entries (siluAVX below dim &^ 7, siluGo past)
-__global__ void flow_sy_kernel(const float *__restrict__ y, const float *__restrict__ tc, int dim,
-                               float *__restrict__ sy) {
+__device__ __forceinline__ void flow_sy(const float *__restrict__ y, const float *__restrict__ tc, int dim, float *sy) {
     for (int j = threadIdx.x; j < dim; j += blockDim.x) {
         const float o = __fadd_rn(y[j], tc[j]);
         const float a = __fdiv_rn(o, __fadd_rn(grx_exp8(__fsub_rn(0.f, o)), 1.f));
@@ -48,23 +47,29 @@ __global__ void flow_sy_kernel(const float *__restrict__ y, const float *__restr
     }
 }
 
-// n = layerNorm(h) (float64 statistics; gain and bias when given), then
-// n*(1+scale) + shift, one workgroup
-__global__ void flow_lnmod_kernel(const float *__restrict__ h, int dim, const float *__restrict__ w,
-                                  const float *__restrict__ b, const float *__restrict__ shift,
-                                  const float *__restrict__ scale, double eps, float *__restrict__ n) {
-    __shared__ double red[48];  // ln_block_reduce
-    __shared__ float hl[8192];  // the row (dim <= 8192, checked at set-up)
-    const int t = threadIdx.x;
-    for (int j = t; j < dim; j += kFT) hl[j] = h[j];
+__global__ void flow_sy_kernel(const float *__restrict__ y, const float *__restrict__ tc, int dim,
+                               float *__restrict__ sy) {
+    flow_sy(y, tc, dim, sy);
+}
+
+// Every ada product of a step: block b of the head (blockIdx.y; the last is
+// the final layer's) gives rows 64 blockIdx.x.. of shift|scale|gate = ada.sy
+// + bias.  They depend on sy only, so one launch forms them all, each
+// workgroup making sy for itself: at dim 512 and six blocks one launch of
+// 168 workgroups where eight (sy's, then 24 workgroups at a time) took 43 us.
+__global__ __launch_bounds__(256) void flow_ada_kernel(const float *__restrict__ y, const float *__restrict__ tc,
+                                                       int dim, int depth, const FlowAda *__restrict__ ada,
+                                                       float *__restrict__ mod) {
+    extern __shared__ __align__(16) float sy[];
+    const int b = blockIdx.y, n = b < depth ? 3 * dim : 2 * dim;
+    if ((int)blockIdx.x * 64 >= n) return;
+    const FlowAda w = ada[b];
+    flow_sy(y, tc, dim, sy);
     __syncthreads();
-    double mean, inv;
-    ln64_stats(hl, dim, eps, red, mean, inv);
-    for (int j = t; j < dim; j += kFT) {
-        float o = (float)__dmul_rn(__dsub_rn((double)hl[j], mean), inv);
-        if (w) o = __fadd_rn(__fmul_rn(o, w[j]), b[j]);
-        n[j] = __fadd_rn(__fmul_rn(o, __fadd_rn(1.f, scale[j])), shift[j]);
-    }
+    int row;
+    bool emit;
+    const float o = q8_float_row(sy, w.qs, w.ds, dim / 32, n, blockIdx.x, row, emit);
+    if (emit) mod[(size_t)b * 3 * dim + row] = __fadd_rn(o, w.bias[row]);
 }
 
 // x += v / steps; on the last step the latent also goes to lat[*frame]
@@ -78,9 +83,9 @@ __global__ void flow_update_kernel(float *__restrict__ cur, const float *__restr
 }
 
 grx_status linear(hipStream_t st, const FlowMat &w, const float *x, const float *bias, float *y,
-                  GrxFloatEpi e = GrxFloatEpi()) {
-    if (w.q8) return grx_float_gemv_q8(st, w.q8, x, bias, y, e);
-    return grx_float_gemv_f32(st, w.f32, w.rows, w.cols, x, bias, y, e);
+                  GrxFloatEpi e = GrxFloatEpi(), GrxFloatPro p = GrxFloatPro()) {
+    if (w.q8) return grx_float_gemv_q8(st, w.q8, x, bias, y, e, p);
+    return grx_float_gemv_f32(st, w.f32, w.rows, w.cols, x, bias, y, e, p);
 }
 
 struct Spec {
@@ -261,10 +266,18 @@ grx_status flow_finalize_tensors(grx_pocket *m) {
     const size_t big = std::max(d, D);
     if ((s = dev(m, (size_t)f.steps * D, &f.tc)) != GRX_OK) return s;
     if ((s = dev(m, (size_t)(m->hp.max_pos + 1) * ld, &f.noise)) != GRX_OK) return s;
-    for (float **b : {&f.y, &f.sy, &f.h, &f.n, &f.mm})
+    for (float **b : {&f.y, &f.sy, &f.h, &f.mm})
         if ((s = dev(m, (size_t)D, b)) != GRX_OK) return s;
     if ((s = dev(m, big + 512 + 2 * (size_t)D, &f.yi)) != GRX_OK) return s;  // c, and time-embedding scratch
-    if ((s = dev(m, 3 * (size_t)D, &f.mod)) != GRX_OK) return s;
+    if ((s = dev(m, (3 * (size_t)f.depth + 2) * D, &f.mod)) != GRX_OK) return s;
+    std::vector<FlowAda> ada;
+    for (const FlowRes &r : f.res)
+        if (r.ada.q8) ada.push_back({r.ada.q8->qs, r.ada.q8->ds, r.ada_b});
+    if (f.final_ada.q8) ada.push_back({f.final_ada.q8->qs, f.final_ada.q8->ds, f.final_ada_b});
+    if ((int)ada.size() == f.depth + 1) {
+        if ((s = dev(m, ada.size(), &f.ada)) != GRX_OK) return s;
+        GRX_HIP(hipMemcpy(f.ada, ada.data(), ada.size() * sizeof(FlowAda), hipMemcpyHostToDevice));
+    }
     if ((s = dev(m, (size_t)ld, &f.cur)) != GRX_OK) return s;
     if ((s = dev(m, (size_t)ld, &f.v)) != GRX_OK) return s;
     // timeConds (lm.go:89-104): the mean of the start and end times' embeddings,
@@ -319,21 +332,36 @@ grx_status pocket_flow_enqueue(grx_pocket *m, hipStream_t st) {
     silu.kind = GRX_FEPI_SILU;
     gate.kind = GRX_FEPI_GATE;
     for (int step = 0; step < f.steps; ++step) {
-        flow_sy_kernel<<<1, kFT, 0, st>>>(f.y, f.tc + (size_t)step * D, D, f.sy);
-        GRX_LAUNCHED("flow_sy_kernel");
-        if ((s = linear(st, f.input, f.cur, f.input_b, f.h)) != GRX_OK) return s;
-        for (FlowRes &r : f.res) {
-            if ((s = linear(st, r.ada, f.sy, r.ada_b, f.mod)) != GRX_OK) return s;
-            flow_lnmod_kernel<<<1, kFT, 0, st>>>(f.h, D, r.norm_w, r.norm_b, f.mod, f.mod + D, 1e-6, f.n);
-            GRX_LAUNCHED("flow_lnmod_kernel");
-            if ((s = linear(st, r.fc1, f.n, r.b1, f.mm, silu)) != GRX_OK) return s;
-            gate.gate = f.mod + 2 * D;
-            if ((s = linear(st, r.fc2, f.mm, r.b2, f.h, gate)) != GRX_OK) return s;
+        const float *tc = f.tc + (size_t)step * D;
+        if (f.ada) {
+            flow_ada_kernel<<<dim3(grx_ceil_div(3 * D, 64), f.depth + 1), 256, (size_t)D * 4, st>>>(f.y, tc, D, f.depth,
+                                                                                                 f.ada, f.mod);
+            GRX_LAUNCHED("flow_ada_kernel");
+        } else {
+            flow_sy_kernel<<<1, kFT, 0, st>>>(f.y, tc, D, f.sy);
+            GRX_LAUNCHED("flow_sy_kernel");
+            for (int i = 0; i <= f.depth; ++i)
+                if ((s = i < f.depth ? linear(st, f.res[i].ada, f.sy, f.res[i].ada_b, f.mod + (size_t)i * 3 * D)
+                                     : linear(st, f.final_ada, f.sy, f.final_ada_b, f.mod + (size_t)i * 3 * D)) !=
+                    GRX_OK)
+                    return s;
         }
-        if ((s = linear(st, f.final_ada, f.sy, f.final_ada_b, f.mod)) != GRX_OK) return s;
-        flow_lnmod_kernel<<<1, kFT, 0, st>>>(f.h, D, nullptr, nullptr, f.mod, f.mod + D, 1e-6, f.n);
-        GRX_LAUNCHED("flow_lnmod_kernel");
-        if ((s = linear(st, f.out, f.n, f.out_b, f.v)) != GRX_OK) return s;
+        if ((s = linear(st, f.input, f.cur, f.input_b, f.h)) != GRX_OK) return s;
+        GrxFloatPro ln;
+        ln.eps = 1e-6;
+        ln.shift = f.mod;
+        for (FlowRes &r : f.res) {
+            ln.scale = ln.shift + D;
+            ln.w = r.norm_w;
+            ln.b = r.norm_b;
+            if ((s = linear(st, r.fc1, f.h, r.b1, f.mm, silu, ln)) != GRX_OK) return s;
+            gate.gate = ln.shift + 2 * D;
+            if ((s = linear(st, r.fc2, f.mm, r.b2, f.h, gate)) != GRX_OK) return s;
+            ln.shift += 3 * D;
+        }
+        ln.scale = ln.shift + D;
+        ln.w = ln.b = nullptr;
+        if ((s = linear(st, f.out, f.h, f.out_b, f.v, GrxFloatEpi(), ln)) != GRX_OK) return s;
         flow_update_kernel<<<1, 64, 0, st>>>(f.cur, f.v, ld, (float)f.steps, step + 1 == f.steps ? m->lat : nullptr,
                                              m->frame);
         GRX_LAUNCHED("flow_update_kernel");

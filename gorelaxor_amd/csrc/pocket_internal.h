@@ -21,6 +21,13 @@ struct FlowRes {
     float *norm_w = nullptr, *norm_b = nullptr, *ada_b = nullptr, *b1 = nullptr, *b2 = nullptr;
 };
 
+// A shift|scale|gate product of the flow head, as one launch makes them all
+struct FlowAda {
+    const int8_t *qs;
+    const uint16_t *ds;
+    const float *bias;
+};
+
 // SimpleMLPAdaLN of pockettts/lm.go:27-53 and its per-frame buffers
 struct FlowHead {
     bool on = false, ready = false;
@@ -28,9 +35,11 @@ struct FlowHead {
     FlowMat cond, input, final_ada, out;
     float *cond_b = nullptr, *input_b = nullptr, *final_ada_b = nullptr, *out_b = nullptr;
     std::vector<FlowRes> res;
+    FlowAda *ada = nullptr;   // [depth + 1] in device memory; NULL unless every one is Q8_0
     float *tc = nullptr;      // [steps][dim] time conditions
     float *noise = nullptr;   // [max_pos][ldim] the caller's noise, one row a frame
-    float *y = nullptr, *yi = nullptr, *sy = nullptr, *h = nullptr, *n = nullptr, *mm = nullptr, *mod = nullptr;
+    float *y = nullptr, *yi = nullptr, *sy = nullptr, *h = nullptr, *mm = nullptr;
+    float *mod = nullptr;     // shift|scale|gate of each block, then the final shift|scale
     float *cur = nullptr, *v = nullptr;
 };
 
