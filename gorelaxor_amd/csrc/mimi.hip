@@ -25,6 +25,7 @@
 
 #include "grx_float.h"
 #include "grx_internal.h"
+#include "grx_quant.h"
 #include "grx_ln.h"
 
 namespace {
@@ -44,6 +45,41 @@ __device__ __forceinline__ float elu_at(float v, size_t i, size_t n) {
     const float t = __fsub_rn(v < 0.f ? v : 0.f, 0.f);
     const float e = (i - c0) < (cl & ~(size_t)7) ? grx_exp8(t) : grx_expf_go(t);
     return __fadd_rn(v > 0.f ? v : 0.f, __fsub_rn(e, 1.f));
+}
+
+// The rows a product takes, made and rounded to Q8_0 in one pass (nothing
+// else reads them): ELU or GELU of n values, or conv.run's columns
+// (ConvRows).  Launches bind here: 16 latents one a call took 4.78 ms with
+// ELU, GELU and columns in passes of their own before the rounding, 4.46 so.
+struct EluRows {
+    const float *x;
+    int k;  // values a row
+    size_t n;
+    __device__ float operator()(int r, int c) const {
+        const size_t i = (size_t)r * k + c;
+        return elu_at(x[i], i, n);
+    }
+};
+struct GeluRows {
+    const float *x;
+    int k;
+    size_t n;
+    __device__ float operator()(int r, int c) const {
+        const size_t i = (size_t)r * k + c;
+        return grx_gelu_at(x[i], (int)i, (int)n);
+    }
+};
+template <typename Rows>
+__global__ __launch_bounds__(kThreads) void round_rows_kernel(const Rows rows, uint32_t blocks, uint32_t nb,
+                                                              int8_t *__restrict__ q, float *__restrict__ sc) {
+    const uint32_t b = blockIdx.x * (kThreads / 8) + (threadIdx.x >> 3);
+    const int l8 = threadIdx.x & 7;
+    if (b >= blocks) return;  // whole groups of eight lanes
+    const int r = (int)(b / nb), c = (int)(b % nb) * GRX_QK + 4 * l8;
+    float v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = rows(r, c + j);
+    quant8x4_store(v, q + (size_t)b * GRX_QK, sc + b, l8);
 }
 
 __global__ void elu_kernel(float *__restrict__ x, size_t n) {
@@ -202,21 +238,21 @@ __global__ void gelu_kernel(float *__restrict__ x, size_t n) {
 // conv.run's im2col (nn.go:283-290): buf = the P carried rows then T rows
 // of x (ELU'd first when elu: runSea's in-place ELU, nn.go/mimi.go:67-69,
 // or the residual block's copy), col row t, tap j = buf row t*stride + j*dil.
-__global__ void im2col_kernel(const float *__restrict__ prev, const float *__restrict__ x, int T, int cin, int k,
-                              int stride, int dil, int P, int elu, float *__restrict__ col) {
-    const int To = T / stride, cols = k * cin;
-    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (size_t)To * cols) return;
-    const int t = (int)(idx / cols), q = (int)(idx % cols), j = q / cin, e = q % cin;
-    const int br = t * stride + j * dil;
-    float v;
-    if (br < P) {
-        v = prev[(size_t)br * cin + e];
-    } else {
+struct ConvRows {
+    const float *prev, *x;
+    int T, cin, k, stride, dil, P, elu;
+    __device__ float operator()(int t, int q) const {
+        const int j = q / cin, e = q % cin;
+        const int br = t * stride + j * dil;
+        if (br < P) return prev[(size_t)br * cin + e];
         const size_t xi = (size_t)(br - P) * cin + e;
-        v = elu ? elu_at(x[xi], xi, (size_t)T * cin) : x[xi];
+        return elu ? elu_at(x[xi], xi, (size_t)T * cin) : x[xi];
     }
-    col[idx] = v;
+};
+__global__ void im2col_kernel(const ConvRows rows, size_t n, float *__restrict__ col) {
+    const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int cols = rows.k * rows.cin;
+    if (idx < n) col[idx] = rows((int)(idx / cols), (int)(idx % cols));
 }
 
 // The carried rows after a conv call: the last P rows of buf (nn.go:293),
@@ -401,11 +437,35 @@ void release(grx_mimi *m) {
 
 void gridn(size_t n, unsigned *blocks) { *blocks = (unsigned)((n + kThreads - 1) / kThreads); }
 
+// Whether lin rounds its rows in a launch of its own (round_rows_kernel can
+// make them then), not in the product's prologue.
+bool lin_rounds(const MLin &w, int rows) { return w.q && !(rows % 8 == 0 && rows <= 64 && w.k <= 1280); }
+
+// The product of rows rounded already (m->xq, m->xs)
+grx_status lin_rounded(grx_mimi *m, hipStream_t st, const MLin &w, int rows, float *y, bool add) {
+    GemmOut o;
+    o.y = y;
+    o.ldc = w.n;
+    o.epi = add ? GRX_GEMM_ADD : GRX_GEMM_STORE;
+    return grx_gemm_q8_launch_ex(st, w.q, m->xq, m->xs, rows, w.b, o);
+}
+
+// The rows of `src` made and rounded, then their product
+template <typename Rows>
+grx_status lin_made(grx_mimi *m, hipStream_t st, const MLin &w, const Rows &src, int rows, float *y, bool add = false) {
+    if (rows == 0) return GRX_OK;
+    const uint32_t nb = w.k / GRX_QK, blocks = rows * nb;  // of the call's buffers: far fewer than 2^31
+    round_rows_kernel<Rows><<<(blocks + kThreads / 8 - 1) / (kThreads / 8), kThreads, 0, st>>>(src, blocks, nb, m->xq,
+                                                                                              m->xs);
+    GRX_LAUNCHED("round_rows_kernel");
+    return lin_rounded(m, st, w, rows, y, add);
+}
+
 // kern.Linear(y, x, rows, w, bias) by the weight's route; ADD (Q8_0 only):
 // y += the product (kern.Add of it, the residual's sum).
 grx_status lin(grx_mimi *m, hipStream_t st, const MLin &w, const float *x, int rows, float *y, bool add = false) {
     if (rows == 0) return GRX_OK;
-    if (w.q && rows % 8 == 0 && rows <= 64 && w.k <= 1280) {
+    if (w.q && !lin_rounds(w, rows)) {
         // a few groups of 8 rows in one several-row GEMV launch that rounds
         // its rows in its own prologue (quantU8, the same arithmetic as the
         // rounding launch it replaces)
@@ -428,11 +488,7 @@ grx_status lin(grx_mimi *m, hipStream_t st, const MLin &w, const float *x, int r
     if (w.q) {
         grx_status s = grx_quant_rows(st, x, w.k, rows, w.k, m->xq, m->xs);
         if (s != GRX_OK) return s;
-        GemmOut o;
-        o.y = y;
-        o.ldc = w.n;
-        o.epi = add ? GRX_GEMM_ADD : GRX_GEMM_STORE;
-        return grx_gemm_q8_launch_ex(st, w.q, m->xq, m->xs, rows, w.b, o);
+        return lin_rounded(m, st, w, rows, y, add);
     }
     if (add) return grx_fail(GRX_EINVAL, "grx_mimi: a float32 residual product adds separately");
     return grx_float_rows_f32(st, x, w.f, w.b, y, 1, rows, w.n, w.k);
@@ -445,13 +501,22 @@ grx_status conv_run(grx_mimi *m, hipStream_t st, MConv &c, const float *x, int T
         return lin(m, st, c.w, x, T, y);
     }
     const int To = T / c.stride;
-    gridn((size_t)To * c.k * c.cin, &blocks);
-    im2col_kernel<<<blocks, kThreads, 0, st>>>(c.prev, x, T, c.cin, c.k, c.stride, c.dil, c.past, elu, m->col);
-    GRX_LAUNCHED("im2col_kernel");
+    const ConvRows src{c.prev, x, T, c.cin, c.k, c.stride, c.dil, c.past, elu};
+    const bool made = lin_rounds(c.w, To);
+    grx_status s = GRX_OK;
+    if (made) {
+        s = lin_made(m, st, c.w, src, To, y);
+    } else {
+        const size_t n = (size_t)To * c.k * c.cin;
+        gridn(n, &blocks);
+        im2col_kernel<<<blocks, kThreads, 0, st>>>(src, n, m->col);
+        GRX_LAUNCHED("im2col_kernel");
+    }
+    if (s != GRX_OK) return s;
     gridn((size_t)c.cin, &blocks);
     conv_past_kernel<<<blocks, kThreads, 0, st>>>(c.prev, x, T, c.cin, c.past, elu);
     GRX_LAUNCHED("conv_past_kernel");
-    return lin(m, st, c.w, m->col, To, y);
+    return made ? GRX_OK : lin(m, st, c.w, m->col, To, y);
 }
 
 // decode (mimi.go:122-152) of n latents at lat (device) into out (device)
@@ -507,10 +572,15 @@ grx_status enqueue_decode(grx_mimi *m, hipStream_t st, const float *lat, int n, 
         ln64_rows_kernel<<<T, kThreads, (size_t)d * 4, st>>>(m->x, d, L.n2w, L.n2b, m->h);
         GRX_LAUNCHED("ln64_rows_kernel");
         if ((s = lin(m, st, L.ff1, m->h, T, m->f)) != GRX_OK) return s;
-        gridn((size_t)T * hp.ff, &blocks);
-        gelu_kernel<<<blocks, kThreads, 0, st>>>(m->f, (size_t)T * hp.ff);
-        GRX_LAUNCHED("gelu_kernel");
-        if ((s = lin(m, st, L.ff2, m->f, T, m->h)) != GRX_OK) return s;
+        if (lin_rounds(L.ff2, T)) {
+            s = lin_made(m, st, L.ff2, GeluRows{m->f, hp.ff, (size_t)T * hp.ff}, T, m->h);
+        } else {
+            gridn((size_t)T * hp.ff, &blocks);
+            gelu_kernel<<<blocks, kThreads, 0, st>>>(m->f, (size_t)T * hp.ff);
+            GRX_LAUNCHED("gelu_kernel");
+            s = lin(m, st, L.ff2, m->f, T, m->h);
+        }
+        if (s != GRX_OK) return s;
         gridn((size_t)T * d, &blocks);
         add_scaled_kernel<<<blocks, kThreads, 0, st>>>(m->x, m->h, L.ls2, d, (size_t)T * d);
         GRX_LAUNCHED("add_scaled_kernel");
@@ -530,12 +600,17 @@ grx_status enqueue_decode(grx_mimi *m, hipStream_t st, const float *lat, int n, 
             std::swap(cur, nxt);
         } else if (q.kind == 1) {
             MConvTr &t = q.t;
-            if (q.elu) {
-                gridn((size_t)R * t.cin, &blocks);
-                elu_kernel<<<blocks, kThreads, 0, st>>>(cur, (size_t)R * t.cin);
-                GRX_LAUNCHED("elu_kernel");
+            if (q.elu && lin_rounds(t.w, R)) {
+                s = lin_made(m, st, t.w, EluRows{cur, t.cin, (size_t)R * t.cin}, R, m->z);
+            } else {
+                if (q.elu) {
+                    gridn((size_t)R * t.cin, &blocks);
+                    elu_kernel<<<blocks, kThreads, 0, st>>>(cur, (size_t)R * t.cin);
+                    GRX_LAUNCHED("elu_kernel");
+                }
+                s = lin(m, st, t.w, cur, R, m->z);
             }
-            if ((s = lin(m, st, t.w, cur, R, m->z)) != GRX_OK) return s;
+            if (s != GRX_OK) return s;
             gridn((size_t)R * t.stride * t.cout, &blocks);
             convtr_overlap_kernel<<<blocks, kThreads, 0, st>>>(m->z, t.b, R, t.stride, t.k, t.cout, t.partial, dst);
             GRX_LAUNCHED("convtr_overlap_kernel");
@@ -545,8 +620,14 @@ grx_status enqueue_decode(grx_mimi *m, hipStream_t st, const float *lat, int n, 
             // v = ELU(copy of x) inside the first conv's im2col; h = ELU(a(v));
             // x += b(h)
             if ((s = conv_run(m, st, q.a, cur, R, 1, m->h)) != GRX_OK) return s;
-            gridn((size_t)R * q.a.cout, &blocks);
-            elu_kernel<<<blocks, kThreads, 0, st>>>(m->h, (size_t)R * q.a.cout);
+            const EluRows src{m->h, q.a.cout, (size_t)R * q.a.cout};
+            if (lin_rounds(q.bb.w, R)) {
+                if ((s = lin_made(m, st, q.bb.w, src, R, cur, true)) != GRX_OK) return s;
+                if (last) GRX_HIP(hipMemcpyAsync(out, cur, (size_t)R * q.bb.cout * 4, hipMemcpyDeviceToDevice, st));
+                continue;
+            }
+            gridn(src.n, &blocks);
+            elu_kernel<<<blocks, kThreads, 0, st>>>(m->h, src.n);
             GRX_LAUNCHED("elu_kernel");
             if (q.bb.w.q) {
                 if ((s = lin(m, st, q.bb.w, m->h, R, cur, true)) != GRX_OK) return s;

@@ -20,6 +20,7 @@
 // (q8_gemv1n.hip).
 #include <mutex>
 
+#include "grx_quant.h"
 #include "q8_gemv_impl.h"
 
 namespace {
@@ -782,20 +783,17 @@ __global__ __launch_bounds__(256) void argmax_finish_kernel(const unsigned long 
 }
 
 // One thread per block: quantU8 of m rows (q8int.go:88-105), signed.
-__global__ void quant_act_kernel(const float *__restrict__ x, int lda, int m, int nb,
-                                 int8_t *__restrict__ q, float *__restrict__ sc) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m * nb) return;
+// Eight lanes a block, 16 bytes a lane (a thread a block touched 64 lines a
+// load: 300 x 4096 4.9 us, 4.3 here).
+__global__ __launch_bounds__(256) void quant_act_kernel(const float *__restrict__ x, int lda, int m, int nb,
+                                                        int8_t *__restrict__ q, float *__restrict__ sc) {
+    const int i = blockIdx.x * 32 + (threadIdx.x >> 3), l8 = threadIdx.x & 7;
+    if (i >= m * nb) return;  // whole groups of eight lanes
     const int r = i / nb, b = i - r * nb;
-    const float *src = x + (size_t)r * lda + b * GRX_QK;
-    float v[GRX_QK];
-#pragma unroll
-    for (int j = 0; j < GRX_QK; ++j) v[j] = src[j];
-    int8_t qq[GRX_QK];
-    sc[i] = grx_quant_block(v, qq);
-    int8_t *d = q + (size_t)r * nb * GRX_QK + b * GRX_QK;
-#pragma unroll
-    for (int j = 0; j < GRX_QK; ++j) d[j] = qq[j];
+    const float *src = x + (size_t)r * lda + b * GRX_QK + 4 * l8;
+    float v[4];
+    __builtin_memcpy(v, src, 16);
+    quant8x4_store(v, q + (size_t)i * GRX_QK, sc + i, l8);
 }
 
 // s[m][rows][nb]: one thread per (activation row, weight row, block).
@@ -1106,7 +1104,7 @@ static grx_status gemv_rows_preq(hipStream_t st, float *dst, int ldc, const int8
 grx_status grx_quant_rows(hipStream_t st, const float *x, int lda, int m, int k, int8_t *q, float *sc) {
     const int nb = k / GRX_QK;
     if (m * nb == 0) return GRX_OK;
-    quant_act_kernel<<<grx_ceil_div(m * nb, 256), 256, 0, st>>>(x, lda, m, nb, q, sc);
+    quant_act_kernel<<<grx_ceil_div(m * nb, 32), 256, 0, st>>>(x, lda, m, nb, q, sc);
     GRX_LAUNCHED("quant_act_kernel");
     return GRX_OK;
 }
@@ -1120,7 +1118,7 @@ extern "C" grx_status grx_quant_act_dev(grx_ctx *ctx, int8_t *q, float *sc, cons
     if (m * nb == 0) return GRX_OK;
     if (!q || !sc || !x) return grx_fail(GRX_EINVAL, "grx_quant_act_dev: NULL buffer");
     GRX_HIP(hipSetDevice(ctx->device));
-    quant_act_kernel<<<grx_ceil_div(m * nb, 256), 256, 0, ctx->stream>>>(x, lda, m, nb, q, sc);
+    quant_act_kernel<<<grx_ceil_div(m * nb, 32), 256, 0, ctx->stream>>>(x, lda, m, nb, q, sc);
     GRX_LAUNCHED("quant_act_kernel");
     return GRX_OK;
 }
