@@ -172,11 +172,18 @@ __global__ void mimi_rope_ring_kernel(float *__restrict__ qkv, int T, int d, int
 // order, block_softmax); then T < 4: AddScaled over the nk = pos0 + T - lo0
 // keys in order, zero weights skipped; else the product of the row with the
 // values by the same route, over all nk keys.  The head's value rows are
-// staged in LDS ([nk][hd]), keys read from the ring.
-__global__ __launch_bounds__(kThreads) void mimi_attn_kernel(const float *__restrict__ qkv, const float *__restrict__ kr,
-                                                             const float *__restrict__ vr, int cap,
-                                                             const long long *__restrict__ posd, int T, int d, int hd,
-                                                             int context, float scale, float *__restrict__ att) {
+// staged in LDS ([nk][vs], vs = hd + 8 where that fits: eight lanes of eight
+// outputs read 64 distinct banks), keys read from the ring.
+//
+// Bound by latency, in one workgroup a CU (its 68 KB of values): with 256
+// threads, a thread a score and 64 threads forming the outputs one chain
+// after another, 16 rows over 265 keys took 20.6 us; 8.6 with 1024
+// threads, 16-byte staging and eight lanes a dot4f32avx (dot8_s).
+constexpr int kAttnThreads = 1024;
+__global__ __launch_bounds__(kAttnThreads) void mimi_attn_kernel(
+    const float *__restrict__ qkv, const float *__restrict__ kr, const float *__restrict__ vr, int cap,
+    const long long *__restrict__ posd, int T, int d, int hd, int vs, int context, float scale,
+    float *__restrict__ att) {
     extern __shared__ __align__(16) float sm[];
     const long long pos0 = *posd;
     const int h = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
@@ -185,24 +192,50 @@ __global__ __launch_bounds__(kThreads) void mimi_attn_kernel(const float *__rest
     const long long p = pos0 + r;
     const long long lo = p - context + 1 > lo0 ? p - context + 1 : lo0;
     const int off = (int)(lo - lo0), ns = (int)(p + 1 - lo);
-    float *V = sm;            // [nk][hd]
-    float *s = V + nk * hd;   // [nk]
+    float *V = sm;            // [nk][vs]
+    float *s = V + nk * vs;   // [nk]
     float *q = s + nk;        // [hd]
     float *part = q + hd;     // block_softmax's 32
+    const int s0 = (int)(lo0 % cap);
+    auto slot = [&](int j) { return (size_t)(s0 + j < cap ? s0 + j : s0 + j - cap) * d + h * hd; };  // nk <= cap
     for (int i = tid; i < hd; i += blockDim.x) q[i] = qkv[(size_t)r * 3 * d + h * hd + i];
-    for (int i = tid; i < nk * hd; i += blockDim.x) {
-        const int j = i / hd, e = i % hd;
-        V[i] = vr[(size_t)((lo0 + j) % cap) * d + h * hd + e];
+    if ((hd & 3) == 0) {  // 16-byte rows
+        const int pc = hd >> 2;
+#pragma unroll 4
+        for (int i = tid; i < nk * pc; i += blockDim.x) {
+            const int j = i / pc, e = 4 * (i - j * pc);
+            *reinterpret_cast<float4 *>(V + j * vs + e) = *reinterpret_cast<const float4 *>(vr + slot(j) + e);
+        }
+    } else {
+        for (int i = tid; i < nk * hd; i += blockDim.x) V[i / hd * vs + i % hd] = vr[slot(i / hd) + i % hd];
     }
     __syncthreads();
-    for (int j = tid; j < nk; j += blockDim.x) {
-        float v = 0.f;
-        if (j >= off && j < off + ns)
-            v = __fmul_rn(matmul_f32_one(q, kr + (size_t)((lo0 + j) % cap) * d + h * hd, 1, hd, r, T, j, nk), scale);
-        s[j] = v;
+    // the row's route in MatMulF32: k6x16's chain, or gemvRows on eight lanes an output
+    const bool chain = T > 16 && r < T / 6 * 6;
+    const int l8 = tid & 7;
+    if (chain) {
+        for (int j = tid; j < nk; j += blockDim.x) {
+            float v = 0.f;
+            if (j >= off && j < off + ns) v = __fmul_rn(matmul_f32_one(q, kr + slot(j), 1, hd, r, T, j, nk), scale);
+            s[j] = v;
+        }
+    } else {
+        for (int j = tid >> 3; j < nk; j += blockDim.x >> 3) {
+            float v = 0.f;
+            if (j >= off && j < off + ns) v = __fmul_rn(dot8_s(q, kr + slot(j), 1, hd, j < (nk & ~3), l8), scale);
+            if (l8 == 0) s[j] = v;
+        }
     }
     __syncthreads();
     block_softmax(s + off, ns, part);
+    float *o_row = att + (size_t)r * d + h * hd;
+    if (T >= 4 && !chain) {
+        for (int e = tid >> 3; e < hd; e += blockDim.x >> 3) {
+            const float o = dot8_s(s, V + e, vs, nk, e < (hd & ~3), l8);
+            if (l8 == 0) o_row[e] = o;
+        }
+        return;
+    }
     const int h8 = hd & ~7;
     for (int e = tid; e < hd; e += blockDim.x) {
         float o;
@@ -211,13 +244,13 @@ __global__ __launch_bounds__(kThreads) void mimi_attn_kernel(const float *__rest
             for (int j = 0; j < nk; ++j) {
                 const float w = s[j];
                 if (w == 0.f) continue;
-                const float v = V[(size_t)j * hd + e];
+                const float v = V[(size_t)j * vs + e];
                 o = e < h8 ? __fmaf_rn(w, v, o) : __fadd_rn(o, __fmul_rn(w, v));
             }
         } else {
-            o = matmul_f32_one(s, V + e, hd, nk, r, T, e, hd);
+            o = matmul_f32_one(s, V + e, vs, nk, r, T, e, hd);
         }
-        att[(size_t)r * d + h * hd + e] = o;
+        o_row[e] = o;
     }
 }
 
@@ -384,15 +417,16 @@ struct grx_mimi {
     float *rope_host = nullptr;   // pinned
     std::vector<float> freqs;
     size_t act_floats = 0, col_floats = 0, z_floats = 0, h_floats = 0, q_bytes = 0, attn_lds = 0;
+    int attn_vs = 0;  // floats from one staged value row to the next
 };
 
 namespace {
 
 // LDS of the attention kernel: a head's value rows over the ring's
 // positions, one query's scores, the query, block_softmax's 32 floats
-size_t attn_lds(const grx_mimi_hparams &hp) {
+size_t attn_lds(const grx_mimi_hparams &hp, int pad = 0) {
     const size_t cap = (size_t)hp.context + (size_t)hp.max_latents * hp.upsample - 1, hd = hp.d / hp.heads;
-    return (cap * hd + cap + hd + 32) * 4;
+    return (cap * (hd + pad) + cap + hd + 32) * 4;
 }
 
 grx_status malloc_dev(grx_mimi *m, size_t bytes, void **out) {
@@ -562,8 +596,9 @@ grx_status enqueue_decode(grx_mimi *m, hipStream_t st, const float *lat, int n, 
         mimi_rope_ring_kernel<<<blocks, kThreads, 0, st>>>(m->qkv, T, d, hd, m->rope, m->rope + (size_t)m->tmax * half,
                                                            L.kr, L.vr, m->cap, m->posd);
         GRX_LAUNCHED("mimi_rope_ring_kernel");
-        mimi_attn_kernel<<<dim3(hp.heads, T), kThreads, m->attn_lds, st>>>(m->qkv, L.kr, L.vr, m->cap, m->posd, T, d,
-                                                                          hd, hp.context, scale, m->att);
+        mimi_attn_kernel<<<dim3(hp.heads, T), kAttnThreads, m->attn_lds, st>>>(m->qkv, L.kr, L.vr, m->cap, m->posd, T,
+                                                                              d, hd, m->attn_vs, hp.context, scale,
+                                                                              m->att);
         GRX_LAUNCHED("mimi_attn_kernel");
         if ((s = lin(m, st, L.out, m->att, T, m->h)) != GRX_OK) return s;
         gridn((size_t)T * d, &blocks);
@@ -770,7 +805,9 @@ grx_status alloc_state(grx_mimi *m) {
     const int d = hp.d, half = m->hd / 2;
     grx_status s;
     m->cap = hp.context + m->tmax - 1;
-    m->attn_lds = attn_lds(hp);
+    const int pad = attn_lds(hp, 8) <= 160 * 1024 ? 8 : 0;
+    m->attn_lds = attn_lds(hp, pad);
+    m->attn_vs = d / hp.heads + pad;
     if (m->attn_lds > 64 * 1024)
         GRX_HIP(hipFuncSetAttribute((const void *)mimi_attn_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)m->attn_lds));
