@@ -16,8 +16,9 @@
 // MFMAs sharing the A fragment); a workgroup of four waves covers 64 x 64.
 // Per block a lane loads 8 bytes of A, 4 x 8 bytes of B (the weight tile
 // layout keeps each row's 32 bytes in two 16-byte halves), four weight scales
-// and four activation scales.  The per-output fold (convert, multiply, fma:
-// 3 VALU ops per output per block) is the bound, not the MFMA: exact
+// and four activation scales.  The per-output fold (convert, multiply, fma; two
+// fmas in the LDS-staged kernel:
+// 2-3 VALU ops per output per block) is the bound, not the MFMA: exact
 // per-block scaling costs that much vector work per 32 multiply-adds.
 #include <cstdint>
 #include <cstdlib>

@@ -38,6 +38,24 @@ def test_tiny_streamed_bit_exact(kern, orc, q8):
     dec.close()
 
 
+@pytest.mark.parametrize("d,heads,context", [(96, 16, 12), (96, 4, 13), (64, 8, 2500), (64, 1, 40)])
+def test_attention_head_widths_bit_exact(kern, orc, d, heads, context):
+    """Heads of 6 (value rows staged a float at a time), 24, 8 (a window whose
+    padded rows would not fit in LDS) and 64 values, one and three latents a
+    call (both routes of MatMulF32): every sample's bits."""
+    hp = dict(MIMI_TINY, d=d, heads=heads, context=context)
+    t = mimi_model(hp, seed=41, q8=True)
+    ref, dec = _pair(orc, hp, t)
+    lat = mimi_latents(hp, 12, seed=42)
+    i = 0
+    for n in (1, 1, 3, 1, 3, 1, 1, 1):
+        want = ref.decode(lat[i:i + n])
+        got = dec.decode(lat[i:i + n])
+        assert _same(got, want), f"latents {i}: max |diff| {np.abs(got - want).max()}"
+        i += n
+    dec.close()
+
+
 @pytest.mark.parametrize("nf", [6, 22, 34])
 def test_float_rows_odd_widths_bit_exact(kern, orc, nf):
     """float32 convolutions whose row lengths are no multiple of 4 (rows read

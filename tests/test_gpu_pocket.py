@@ -173,6 +173,16 @@ def test_speak_frames_with_flow_head_bit_exact(kern, orc, q8):
     _speak_check(lm, ref, flow, hp, prefix=5, frames=7, seed=14, chunks=2)
 
 
+@pytest.mark.parametrize("dim,depth,steps", [(96, 1, 3), (32, 3, 2), (160, 5, 1)])
+def test_speak_flow_head_widths_bit_exact(kern, orc, dim, depth, steps):
+    """Flow heads whose shift|scale|gate rows end within a 64-row tile (288,
+    96 and 480 rows, the final layer's 192, 64 and 320), one to five blocks,
+    several steps a frame: every latent's bits."""
+    hp, fhp = dict(POCKET_TTS_TINY), dict(dim=dim, depth=depth, steps=steps)
+    lm, ref, flow = _speak_pair(orc, hp, fhp, seed=23 + dim)
+    _speak_check(lm, ref, flow, hp, prefix=3, frames=5, seed=24, chunks=2)
+
+
 def test_speak_configured_shape(kern, orc):
     """d 1024 transformer with a 512-wide, 6-block flow head (one LSD step):
     a 64-row prefix, then 12 frames, bit-identical."""
