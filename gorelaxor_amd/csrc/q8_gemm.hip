@@ -926,12 +926,19 @@ __global__ __launch_bounds__(64 * WM *WN, FR *FC == 4 ? 4 : 2) void gemm_q8_lds_
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN;  // wave rows 16 FR wm.., columns 16 FC wn..
-    // Workgroup i runs on XCD i % 8: each XCD takes one run of the tiles,
-    // row groups of a column group together, so that a column group's
-    // weights come into one L2
-    const int nrg = (m + T::TM - 1) / T::TM, total = gridDim.x;
+    // Workgroup i runs on XCD i % 8: each XCD takes one run of the tiles, row
+    // groups of a column group together, so that a column group's weights
+    // come into one L2; or, from a quarter as many activation rows as weight
+    // rows on, the column groups of a row group together, so that an L2 reads
+    // its eighth of the activations and every weight (2016 x 1024 x 1024
+    // 18.1 us by columns, 16.5 by rows, 1500 x 2048 x 1024 22.4 and 21.4,
+    // 2016 x 2048 x 480 16.1 and 15.1; 500 x 4096 x 1024 15.4 and 15.9, 200
+    // x 16384 x 1024 21.2 and 23.2)
+    const bool byrow = (long)m * 4 > rows;
+    const int nrg = (m + T::TM - 1) / T::TM, ncg = (rows + T::TN - 1) / T::TN, total = gridDim.x;
     const int xcd = blockIdx.x & 7, id = xcd * (total >> 3) + min(xcd, total & 7) + (blockIdx.x >> 3);
-    const int mb = (id % nrg) * T::TM, nc = (id / nrg) * T::TN;  // activation rows mb.., weight rows nc..
+    const int per = byrow ? ncg : nrg, lo = id % per, hi = id / per;
+    const int mb = (byrow ? hi : lo) * T::TM, nc = (byrow ? lo : hi) * T::TN;  // activation rows mb.., weight rows nc..
     const int K = nb * GRX_QK;
     const int li = lane & 15, lk = lane >> 4;
     if (tid == 0) odd = 0;

@@ -286,11 +286,14 @@ def test_matmul_lds_tiles_and_register_tiles(kern, orc, kernel):
                 _check_matmul(kern, orc, rng, m, n, 32 * nb, bias=(m % 2 == 1))
 
 
-@pytest.mark.parametrize("m,n", [(65, 9217), (140, 5800), (65, 2081), (97, 2050), (65, 300), (33, 33)])
+@pytest.mark.parametrize("m,n", [(65, 9217), (140, 5800), (65, 2081), (97, 2050), (65, 300), (33, 33), (1155, 1290),
+                                 (700, 380), (300, 290)])
 def test_matmul_lds_each_tile(kern, orc, m, n):
     """The LDS-staged product's tiles (64 x 128, 64 x 32, 32 x 32, by the
-    number of tiles), over block counts around one and two copies of blocks:
-    bit-identical to the oracle."""
+    number of tiles) in both orders over the XCDs (by columns below a quarter
+    as many activation rows as weight rows, by rows from there on; tile counts
+    that are and are no multiple of eight), over block counts around one and
+    two copies of blocks: bit-identical to the oracle."""
     rng = np.random.default_rng(59 + n)
     with kern.tuned(GEMM_KERNEL=3):
         for nb in (1, 3, 4, 5, 8, 9, 16, 17, 21):
