@@ -1483,18 +1483,23 @@ void launch_lds(hipStream_t st, const grx_weight *w, const int8_t *xq, const flo
 // give more workgroups: 1024 x 4096 6.2 us on 128 workgroups of 8 rows
 // against 8.0 K-split; a forced GEMM_KERNEL keeps the matrix cores); the
 // LDS-staged tiles from 256 rows on, and from 33 where 64 x 32 tiles of the
-// output are 128 or more (calls with the rounding launch: 126 x 4096 x 1024
-// 10.5 us against 12.3 K-split, 126 x 2048 x 1024 8.8 against 9.8, 240 x 1024
-// x 4096 17.6 against 21.0, 48 x 4096 x 1024 8.9 against 9.8; with 64 tiles
-// the K-split wins: 126 x 1024 x 4096 13.8 against 16.4); below that the
-// K-split tiles with their activations staged through LDS (at 224 rows: 1024
-// x 4096 17 us against 26 on the whole-K register walk); without the
-// staging, the K-split tiles up to 128 rows where the register walk has few
-// tiles or a long K (at 126 rows: 4096 x 1024 10.4 us on the register walk
-// against 11.9 K-split; 2048 x 1024 8.1 against 7.3; 1024 x 4096 25 against
-// 19), the register walk otherwise.  The K-split kernel stages the
-// activations through LDS unless told not to or they are not in 16-byte
-// aligned whole groups of four blocks (a fused prologue builds them there).
+// output are 128 or more or the K-split kernel does not take the product
+// (calls with the rounding launch: 126 x 4096 x 1024 10.5 us against 12.3
+// K-split, 126 x 2048 x 1024 8.8 against 9.8, 240 x 1024 x 4096 17.6 against
+// 21.0, 48 x 4096 x 1024 8.9 against 9.8; with 64 tiles the K-split wins: 126
+// x 1024 x 4096 13.8 against 16.4; blocks in no groups of four: 33 x 4096 x
+// 1056 7.8 against 8.3 on the register walk, 255 x 16384 x 480 15.1 against
+// 24.0; more blocks than a K-split workgroup holds: 100 x 1280 x 5120 18.1
+// against 33.0, 40 x 64 x 4640 16.4 against 22.6); below that the K-split
+// tiles with their activations staged through LDS (at 224 rows: 1024 x 4096
+// 17 us against 26 on the whole-K register walk); without the staging, the
+// K-split tiles up to 128 rows where the register walk had few tiles or a
+// long K (at 126 rows: 2048 x 1024 8.1 us on it against 7.3 K-split, 1024 x
+// 4096 25 against 19).  The register walk is left for up to 32 rows of more
+// blocks than the K-split kernel takes, with no carry to run them in turns.
+// The K-split kernel stages the activations through LDS unless told not to or
+// they are not in 16-byte aligned whole groups of four blocks (a fused
+// prologue builds them there).
 enum Route { kRouteGemv1, kRouteLds, kRouteKs, kRouteMfma };
 struct RoutePick {
     Route r;
@@ -1514,7 +1519,7 @@ RoutePick pick_route(const grx_weight *w, const int8_t *xq, const float *xs, int
     p.sa = grx_tune(GRX_TUNE_GEMM_STAGE_A) != 0 && p.da4 && (pro || ((uintptr_t)xq & 15) == 0);
     const bool ks_ok = pick_ks(m, w->nb, w->rows, o.epi, o.carry != nullptr, p.sa, pro, &p.ns, &p.kb) &&
                        (kind == 2 || (p.sa ? m < 256 : (m <= 128 && (m <= 32 || w->rows <= 2048 || w->nb > 64))));
-    const bool lds = m >= 256 || (m > 32 && p.sa && !pro && grx_ceil_div(m, 64) * grx_ceil_div(w->rows, 32) >= 128);
+    const bool lds = m >= 256 || (m > 32 && !pro && (!ks_ok || grx_ceil_div(m, 64) * grx_ceil_div(w->rows, 32) >= 128));
     if (kind == 3 || (kind != 1 && kind != 2 && lds)) {
         p.r = kRouteLds;
     } else if (kind != 1 && ks_ok) {

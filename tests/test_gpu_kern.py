@@ -6,6 +6,7 @@ Structure follows the reference tests (internal/kern/q8int_test.go,
 odd_test.go, kern_test.go of github.com/xattribution/gorelaxor).
 """
 import os
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -298,6 +299,36 @@ def test_matmul_lds_each_tile(kern, orc, m, n):
     with kern.tuned(GEMM_KERNEL=3):
         for nb in (1, 3, 4, 5, 8, 9, 16, 17, 21):
             _check_matmul(kern, orc, rng, m, n, 32 * nb, bias=(nb % 2 == 1))
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 4100, 1056), (64, 2080, 96), (129, 64, 1056), (255, 100, 480), (40, 64, 4640),
+                                   (200, 100, 5120), (33, 33, 4128), (32, 64, 4640), (128, 2048, 1056)])
+def test_matmul_33_to_255_rows_bit_exact(kern, orc, m, n, k):
+    """Rows below the LDS-staged tiles' usual 256 whose blocks come in no
+    groups of four, or are more than a K-split workgroup holds (128), by the
+    choice a call makes itself: bit-identical to the oracle."""
+    _check_matmul(kern, orc, np.random.default_rng(m + n + k), m, n, k, bias=(m % 2 == 1))
+
+
+@pytest.mark.parametrize("off", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("m,n,k", [(40, 4200, 96), (100, 2100, 256), (200, 80, 4640), (300, 200, 288), (200, 300, 1024)])
+def test_matmul_prequant_alignment(kern, orc, dev, m, n, k, off):
+    """Rounded activations that start `off` bytes past a 256-byte boundary
+    (the entry asks for no alignment of them): bit-identical to the oracle."""
+    rng = np.random.default_rng(off + m)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    w8 = q8_weight(rng, n, k)
+    w = kern.NewQ8(n, k, w8)
+    dx = dev.DeviceBuffer.from_array(x)
+    dq, ds = dev.DeviceBuffer(m * k + 256), dev.DeviceBuffer(m * (k // QK) * 4)
+    dy = dev.DeviceBuffer(m * n * 4)
+    at = SimpleNamespace(data_ptr=lambda: dq.ptr + off)
+    kern.quant_act_dev(at, ds, dx, m, k)
+    kern.matmul_prequant_dev(dy, at, ds, m, w)
+    kern.default_context().sync()
+    got = dy.download(np.float32, (m, n))
+    want = orc.matmul_q8_int(x, w8, n, k, None)
+    assert _bits_equal(got, want), _report(got, want)
 
 
 @pytest.mark.parametrize("m,n", [(65, 9217), (65, 2081), (65, 300)])
