@@ -1300,12 +1300,15 @@ grx_status run_prompt(grx_whisper *m, const int32_t *prompts, int n) {
         for (int k = 0; k < S; ++k)
             order.insert(order.end(), prompts + (size_t)k * n + i, prompts + (size_t)k * n + std::min(n, i + most));
     GRX_HIP(hipMemcpyAsync(m->pr_tok, order.data(), order.size() * 4, hipMemcpyHostToDevice, stream));
-    for (int i = 0; i < n; i += most) {
+    for (int i = 0; i < n && s == GRX_OK; i += most) {
         const int per = std::min(most, n - i);
-        if ((s = enqueue_prompt(m, stream, m->pr_tok + (size_t)S * i, per, i + per == n)) != GRX_OK) return s;
-        m->pos_host += per;
+        s = enqueue_prompt(m, stream, m->pr_tok + (size_t)S * i, per, i + per == n);
+        if (s == GRX_OK) m->pos_host += per;
     }
-    GRX_HIP(hipStreamSynchronize(stream));  // order is read by the copy
+    // the copy reads order: wait for it, after a failed pass too
+    const hipError_t e = hipStreamSynchronize(stream);
+    if (s != GRX_OK) return s;
+    GRX_HIP(e);
     return GRX_OK;
 }
 
