@@ -909,8 +909,8 @@ struct grx_whisper {
     unsigned long long *keys = nullptr;  // argmax keys, [vocabulary tiles][streams]
     unsigned int *counter = nullptr;
     int *tok = nullptr, *pos = nullptr, *hist = nullptr;
-    // a prompt's rows (grown to the largest prompt: pr_cap rows)
-    int pr_cap = 0;
+    // a prompt's rows: pr_rows of them a pass (0: prompts go token by token)
+    int pr_rows = 0;
     int *pr_tok = nullptr;
     float *pr_x = nullptr, *pr_y = nullptr, *pr_q = nullptr, *pr_as = nullptr, *pr_fs = nullptr;
     int8_t *pr_aq = nullptr, *pr_fq = nullptr;
@@ -996,6 +996,28 @@ void wrelease(grx_whisper *m) {
 }
 
 grx_status finalize_tensors(grx_whisper *m);
+
+// The workspace of prompts decoded as rows of many-row products (heads of
+// 64, a row group's cross scores in LDS; else prompts go token by token), all
+// streams together, made with the step's buffers so that a decode allocates
+// nothing.
+constexpr int kPromptRows = 256;
+grx_status prompt_alloc(grx_whisper *m) {
+    const size_t R = kPromptRows, st = m->hp.n_state;
+    grx_status s;
+    m->pr_rows = 0;
+    if (!grx_cross_prompt_ok(m->hp.n_audio_ctx, m->hp.n_state / m->hp.n_head)) return GRX_OK;
+    if ((s = dev_alloc_t(m, (size_t)m->S * m->hp.n_text_ctx, &m->pr_tok)) != GRX_OK) return s;
+    if ((s = dev_alloc_t(m, R * st, &m->pr_x)) != GRX_OK) return s;
+    if ((s = dev_alloc_t(m, R * 3 * st, &m->pr_y)) != GRX_OK) return s;
+    if ((s = dev_alloc_t(m, R * st, &m->pr_q)) != GRX_OK) return s;
+    if ((s = dev_alloc_t(m, R * st, &m->pr_aq)) != GRX_OK) return s;
+    if ((s = dev_alloc_t(m, R * st / 32, &m->pr_as)) != GRX_OK) return s;
+    if ((s = dev_alloc_t(m, R * 4 * st, &m->pr_fq)) != GRX_OK) return s;
+    if ((s = dev_alloc_t(m, R * 4 * st / 32, &m->pr_fs)) != GRX_OK) return s;
+    m->pr_rows = kPromptRows;
+    return GRX_OK;
+}
 
 grx_status finalize(grx_whisper *m) {
     if (m->ready) return GRX_OK;
@@ -1087,6 +1109,7 @@ grx_status finalize_tensors(grx_whisper *m) {
     if ((s = dev_alloc_t(m, S, &m->tok)) != GRX_OK) return s;
     if ((s = dev_alloc_t(m, 1, &m->pos)) != GRX_OK) return s;
     if ((s = dev_alloc_t(m, S * hp.n_text_ctx, &m->hist)) != GRX_OK) return s;
+    if ((s = prompt_alloc(m)) != GRX_OK) return s;
     GRX_HIP(hipMemset(m->pos, 0, 4));
     GRX_HIP(hipMemset(m->tok, 0, 4 * S));
     m->host.clear();
@@ -1202,36 +1225,13 @@ grx_status launch_self_attn(grx_whisper *m, hipStream_t stream, const WLayer &L,
     return GRX_OK;
 }
 
-// Rows of a prompt decoded in one pass (all streams together; the workspace
-// is sized for them), and the fewest positions that take it: a pass is about
-// 80 launches of ~5 us at base.en, a step 0.22 ms (a 4-token prompt and 96
-// steps: 22.12 ms as steps, 21.93 with the prompt in a pass; 8 streams of
-// large-v3-turbo 48.7 and 47.2).
-constexpr int kPromptRows = 256;
+// The fewest positions that take a pass of rows: a pass is about 80 launches
+// of ~5 us at base.en, a step 0.22 ms (a 4-token prompt and 96 steps: 22.12 ms
+// as steps, 21.93 with the prompt in a pass; 8 streams of large-v3-turbo 48.7
+// and 47.2).
 constexpr int kPromptMin = 3;
 
-// Whether prompts run as rows of many-row products (heads of 64, a row
-// group's cross scores in LDS); else, or tuned off, token by token.
-bool prompt_rows_ok(const grx_whisper *m) {
-    const grx_whisper_hparams &hp = m->hp;
-    return !tuned_off(GRX_TUNE_PROMPT_ROWS) && grx_cross_prompt_ok(hp.n_audio_ctx, hp.n_state / hp.n_head);
-}
-
-grx_status prompt_alloc(grx_whisper *m) {
-    if (m->pr_cap > 0) return GRX_OK;
-    const size_t R = kPromptRows, st = m->hp.n_state;
-    grx_status s;
-    if (!m->pr_tok && (s = dev_alloc_t(m, (size_t)m->S * m->hp.n_text_ctx, &m->pr_tok)) != GRX_OK) return s;
-    if (!m->pr_x && (s = dev_alloc_t(m, R * st, &m->pr_x)) != GRX_OK) return s;
-    if (!m->pr_y && (s = dev_alloc_t(m, R * 3 * st, &m->pr_y)) != GRX_OK) return s;
-    if (!m->pr_q && (s = dev_alloc_t(m, R * st, &m->pr_q)) != GRX_OK) return s;
-    if (!m->pr_aq && (s = dev_alloc_t(m, R * st, &m->pr_aq)) != GRX_OK) return s;
-    if (!m->pr_as && (s = dev_alloc_t(m, R * st / 32, &m->pr_as)) != GRX_OK) return s;
-    if (!m->pr_fq && (s = dev_alloc_t(m, R * 4 * st, &m->pr_fq)) != GRX_OK) return s;
-    if (!m->pr_fs && (s = dev_alloc_t(m, R * 4 * st / 32, &m->pr_fs)) != GRX_OK) return s;
-    m->pr_cap = kPromptRows;
-    return GRX_OK;
-}
+bool prompt_rows_ok(const grx_whisper *m) { return m->pr_rows > 0 && !tuned_off(GRX_TUNE_PROMPT_ROWS); }
 
 // `per` prompt positions of every stream at once, from the position the
 // device holds: the step's graph with S * per rows in every product
@@ -1288,12 +1288,11 @@ grx_status enqueue_prompt(grx_whisper *m, hipStream_t stream, const int *tok, in
 }
 
 // n prompt positions of every stream (prompts [S][n]) from the position
-// reached, in passes of at most kPromptRows rows.
+// reached, in passes of at most pr_rows rows.
 grx_status run_prompt(grx_whisper *m, const int32_t *prompts, int n) {
-    const int S = m->S, most = kPromptRows / S;
+    const int S = m->S, most = m->pr_rows / S;
     hipStream_t stream = m->ctx->stream;
-    grx_status s = prompt_alloc(m);
-    if (s != GRX_OK) return s;
+    grx_status s = GRX_OK;
     std::vector<int32_t> order;  // each pass's tokens as its rows are
     order.reserve((size_t)S * n);
     for (int i = 0; i < n; i += most)
@@ -1666,6 +1665,7 @@ static grx_status check_ready(grx_whisper *m, const char *fn) {
     grx_status s = finalize(m);
     if (s != GRX_OK) return s;
     if (!m->have_cross) return grx_fail(GRX_ESTATE, "%s: no encoder output set", fn);
+    GRX_HIP(hipSetDevice(m->ctx->device));
     return GRX_OK;
 }
 
@@ -1741,7 +1741,7 @@ extern "C" grx_status grx_whisper_greedy_streams(grx_whisper *m, const int32_t *
             return grx_fail(GRX_EINVAL, "grx_whisper_greedy_streams: token %d out of the vocabulary", prompts[i]);
     if ((s = grx_whisper_reset(m)) != GRX_OK) return s;
     hipStream_t stream = m->ctx->stream;
-    // the prompt position by position, every stream's token uploaded first
+    // the prompt as rows, or position by position, every stream's token uploaded first
     std::vector<int32_t> col(S);
     const bool rows = n_prompt >= kPromptMin && prompt_rows_ok(m);
     if (rows && (s = run_prompt(m, prompts, n_prompt)) != GRX_OK) return s;

@@ -159,6 +159,33 @@ def test_whisper_decode():
     assert n > 20
 
 
+@pytest.mark.parametrize("n", [3, 20, 300])
+def test_whisper_prompt_allocates_nothing(n):
+    """A model that is set up decodes prompts of every length with no
+    allocation: with the next one made to fail, one token, then a prompt
+    that runs as rows, give the tokens of a model that had memory."""
+    from gorelaxor_amd.synth import WHISPER_TINY_TEST, encoder_output, whisper_model
+    from gorelaxor_amd.whisper import WhisperDecoder
+
+    hp = dict(WHISPER_TINY_TEST, n_text_ctx=320)
+    t = whisper_model(hp, seed=53)
+    enc = encoder_output(hp, seed=54)
+    prompt = np.random.default_rng(n).integers(0, hp["n_vocab"], n).tolist()
+    toks = []
+    for fail in (False, True):
+        dec = WhisperDecoder(hp, t)
+        try:
+            dec.set_encoder_output(enc)
+            if fail:
+                _arm(0)
+            toks.append([list(dec.greedy(prompt[:1], 2)), list(dec.greedy(prompt, 6))])
+            assert _left() == (0 if fail else -1)
+        finally:
+            _arm(-1)
+            dec.close()
+    assert toks[0] == toks[1]
+
+
 def test_pocket_frames_and_speak():
     from gorelaxor_amd.pocket import PocketLM
     from gorelaxor_amd.synth import POCKET_FLOW_TINY, POCKET_TTS_TINY, pocket_flow_model, pocket_inputs, \
