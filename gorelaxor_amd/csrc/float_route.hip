@@ -180,14 +180,11 @@ hipError_t launch_rows(hipStream_t st, const float *x, const float *w, const flo
     const bool vec = k % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
     auto kern = vec ? f32_rows_mfma_kernel<WR, WC, RF, CF, KC, true> : f32_rows_mfma_kernel<WR, WC, RF, CF, KC, false>;
     if constexpr (T::lds > 64 * 1024) {
-        static const hipError_t ok = [] {
-            const hipError_t e = hipFuncSetAttribute((const void *)f32_rows_mfma_kernel<WR, WC, RF, CF, KC, true>,
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::lds);
-            return e != hipSuccess ? e
-                                   : hipFuncSetAttribute((const void *)f32_rows_mfma_kernel<WR, WC, RF, CF, KC, false>,
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::lds);
-        }();
-        if (ok != hipSuccess) return ok;
+        static GrxDeviceOnce once;
+        const hipError_t e = grx_raise_lds(once, {(const void *)f32_rows_mfma_kernel<WR, WC, RF, CF, KC, true>,
+                                                  (const void *)f32_rows_mfma_kernel<WR, WC, RF, CF, KC, false>},
+                                           T::lds);
+        if (e != hipSuccess) return e;
     }
     kern<<<dim3((n + T::TN - 1) / T::TN, (rows + T::TM - 1) / T::TM), T::NT, T::lds, st>>>(x, w, bias, y, rows, n, k);
     return hipGetLastError();

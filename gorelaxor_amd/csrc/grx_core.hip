@@ -41,6 +41,18 @@ hipError_t grx_pinned_malloc(void **p, size_t bytes) {
     return hipHostMalloc(p, bytes, hipHostMallocDefault);
 }
 
+hipError_t grx_raise_lds(GrxDeviceOnce &once, std::initializer_list<const void *> kernels, size_t bytes) {
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    once.run(device, [&] {
+        for (const void *k : kernels)
+            if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        return e == hipSuccess;
+    });
+    return e;
+}
+
 extern "C" void grx_debug_fail_alloc_after(long long n) { g_alloc_countdown.store(n < 0 ? -1 : n); }
 
 extern "C" long long grx_debug_alloc_countdown(void) { return g_alloc_countdown.load(); }

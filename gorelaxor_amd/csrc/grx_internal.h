@@ -11,7 +11,10 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <initializer_list>
+
 #include "../../include/grx.h"
+#include "grx_once.h"
 
 // ---------------------------------------------------------------- host side
 
@@ -154,6 +157,9 @@ hipError_t grx_pinned_malloc(void **p, size_t bytes);
 // current device, once (grx_ctx_create calls it)
 void grx_noalloc_setup(int device);
 grx_status grx_ctx_scratch(grx_ctx *ctx, size_t bytes, void **out);
+// The kernels' dynamic LDS limit set to `bytes` on the current device, once
+// for each device (hipSuccess when it is set already).
+hipError_t grx_raise_lds(GrxDeviceOnce &once, std::initializer_list<const void *> kernels, size_t bytes);
 
 #define GRX_HIP(expr)                                                       \
     do {                                                                    \

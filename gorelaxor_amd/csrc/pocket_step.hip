@@ -659,14 +659,8 @@ grx_status enqueue_frame(grx_pocket *m, hipStream_t st, const float *lat_base, c
     size_t smem = (32 + (((size_t)hp.max_pos + 3) & ~(size_t)3) + (size_t)rc * hd) * 4;
     if (hd == kStepHd) {
         smem = std::max(smem, kStepLds * 4);
-        static bool raised = false;  // set by the eager frame that precedes any capture
-        if (!raised) {
-            raised = true;
-            GRX_HIP(hipFuncSetAttribute((const void *)attn_step_kernel<true>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kStepLds * 4)));
-            GRX_HIP(hipFuncSetAttribute((const void *)attn_step_kernel<false>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kStepLds * 4)));
-        }
+        static GrxDeviceOnce once;  // set by the eager frame that precedes any capture
+        GRX_HIP(grx_raise_lds(once, {(const void *)attn_step_kernel<true>, (const void *)attn_step_kernel<false>}, kStepLds * 4));
     }
     for (int li = 0; li < hp.n_layer; ++li) {
         PLayer &L = m->L[li];

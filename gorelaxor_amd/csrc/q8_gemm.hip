@@ -1303,18 +1303,15 @@ bool pick_ks(int m, int nb, int rows, int epi, bool carry, bool sa, bool pro, in
     return true;
 }
 
-// Whether the staged-activation instantiation may take its LDS (asked once;
-// more than 64 KB needs the attribute).
+// Whether the staged-activation instantiation may take its LDS (asked once
+// a device; more than 64 KB needs the attribute).
 template <int EPI, int NS, int KB, int PRO>
 bool ks_stage_ok() {
-    static const bool ok = [] {
-        const int need = ks_max_waves(NS, KB) * kss_bytes(KB);
-        const bool r = need <= 64 * 1024 ||
-                       hipFuncSetAttribute((const void *)gemm_q8_kss_kernel<EPI, NS, KB, PRO>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, need) == hipSuccess;
-        (void)hipGetLastError();
-        return r;
-    }();
+    constexpr int need = ks_max_waves(NS, KB) * kss_bytes(KB);
+    if constexpr (need <= 64 * 1024) return true;
+    static GrxDeviceOnce once;
+    const bool ok = grx_raise_lds(once, {(const void *)gemm_q8_kss_kernel<EPI, NS, KB, PRO>}, need) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
     return ok;
 }
 

@@ -827,12 +827,8 @@ template <int M, int W, int PRO, int EPI>
 hipError_t launch_one(hipStream_t st, const GemvArgs &a, int tiles) {
     const size_t smem = gemv_smem(M, W, PRO, a.nb);
     if (smem > 64 * 1024) {
-        static bool raised = false;
-        if (!raised) {
-            raised = true;
-            (void)hipFuncSetAttribute((const void *)gemv_q8_kernel<M, W, PRO, EPI>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        }
+        static GrxDeviceOnce once;
+        (void)grx_raise_lds(once, {(const void *)gemv_q8_kernel<M, W, PRO, EPI>}, 160 * 1024);
     }
     gemv_q8_kernel<M, W, PRO, EPI><<<dim3(tiles, 1, a.chunks > 1 ? a.chunks : 1), 64 * W, smem, st>>>(a);
     return hipGetLastError();
@@ -853,12 +849,8 @@ template <int W, int NP, int PRO, int EPI>
 hipError_t launch1_one(hipStream_t st, const GemvArgs &a, int tiles) {
     const size_t smem = gemv1_smem(W, PRO, a.nb, EPI);
     if (smem > 64 * 1024) {
-        static bool raised = false;
-        if (!raised) {
-            raised = true;
-            (void)hipFuncSetAttribute((const void *)gemv1_kernel<W, NP, PRO, EPI>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        }
+        static GrxDeviceOnce once;
+        (void)grx_raise_lds(once, {(const void *)gemv1_kernel<W, NP, PRO, EPI>}, 160 * 1024);
     }
     const dim3 grid(tiles, EPI == GRX_EPI_XSCORES ? grx_ceil_div(a.nctx, 64) : 1);
     gemv1_kernel<W, NP, PRO, EPI><<<grid, 64 * W, smem, st>>>(a);

@@ -194,12 +194,8 @@ template <int NP, int PRO, int EPI>
 hipError_t launch1n_one(hipStream_t st, const GemvArgs &a, int tiles, int lr) {
     const size_t smem = gemv1n_smem(lr, PRO, a.nb);
     if (smem > 64 * 1024) {
-        static bool raised = false;
-        if (!raised) {
-            raised = true;
-            (void)hipFuncSetAttribute((const void *)gemv1n_kernel<NP, PRO, EPI>,
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        }
+        static GrxDeviceOnce once;
+        (void)grx_raise_lds(once, {(const void *)gemv1n_kernel<NP, PRO, EPI>}, 160 * 1024);
     }
     const int S = 64 >> lr, groups = grx_ceil_div(tiles, 8) * 8 * S;
     int W = gemv1n_waves(a.nb, lr);

@@ -215,8 +215,9 @@ __global__ __launch_bounds__(kPcThreads) void cross_prompt_kernel(
 
 bool grx_cross_prompt_ok(int nctx, int hd) {
     if (hd != kPcHd || pc_lds(nctx) > 160 * 1024) return false;
-    static const bool ok = hipFuncSetAttribute((const void *)cross_prompt_kernel,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) == hipSuccess;
+    static GrxDeviceOnce once;
+    const bool ok = grx_raise_lds(once, {(const void *)cross_prompt_kernel}, 160 * 1024) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
     return ok;
 }
 

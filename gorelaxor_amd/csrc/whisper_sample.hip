@@ -503,13 +503,9 @@ template <int CH>
 grx_status launch_ch(hipStream_t st, const float *logits, const GrxSampleArgs &a, const int *suppress, float *scratch,
                      GrxSampleOut *out, const GrxLoopArgs &la) {
     const size_t smem = sizeof(SampleShared);
-    static bool attr = false;
-    if (!attr) {
-        if (hipFuncSetAttribute((const void *)sample_kernel<CH>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)smem) != hipSuccess)
-            return grx_fail(GRX_EDEVICE, "whisper sampler: %zu bytes of LDS refused", smem);
-        attr = true;
-    }
+    static GrxDeviceOnce once;
+    if (grx_raise_lds(once, {(const void *)sample_kernel<CH>}, smem) != hipSuccess)
+        return grx_fail(GRX_EDEVICE, "whisper sampler: %zu bytes of LDS refused", smem);
     float *vg = scratch, *g = scratch + (size_t)kThreads * CH;
     sample_kernel<CH><<<1, kThreads, smem, st>>>(logits, a, suppress, vg, g, out, la);
     GRX_LAUNCHED("sample_kernel");

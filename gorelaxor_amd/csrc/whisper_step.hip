@@ -1136,12 +1136,8 @@ bool tuned_off(int id) { return grx_tune(id) == 0; }
 // One stream's fused q|k|v + self-attention of every head (qkv_attn_kernel).
 template <int NP, int PRO>
 grx_status launch_qkv_attn(hipStream_t stream, const GemvArgs &a, int nh, float sc, int ctx_rows, grx_whisper *m) {
-    static bool raised = false;  // set by the eager step that precedes any capture
-    if (!raised) {
-        raised = true;
-        GRX_HIP(hipFuncSetAttribute((const void *)qkv_attn_kernel<NP, PRO>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    160 * 1024));
-    }
+    static GrxDeviceOnce once;  // set by the eager step that precedes any capture
+    GRX_HIP(grx_raise_lds(once, {(const void *)qkv_attn_kernel<NP, PRO>}, 160 * 1024));
     qkv_attn_kernel<NP, PRO><<<nh, 1024, qkv_attn_lds(a.nb).total, stream>>>(a, sc, ctx_rows, m->att, m->att_q,
                                                                                m->att_s);
     GRX_LAUNCHED("qkv_attn_kernel");
@@ -1203,14 +1199,8 @@ grx_status launch_self_attn(grx_whisper *m, hipStream_t stream, const WLayer &L,
     size_t smem = (32 + (((size_t)hp.n_text_ctx + 3) & ~(size_t)3) + (size_t)rc * hd) * 4;
     if (hd == kSmallHd) {
         smem = std::max(smem, kSmallLds * 4);
-        static bool raised = false;  // set by the eager step that precedes any capture
-        if (!raised) {
-            raised = true;
-            GRX_HIP(hipFuncSetAttribute((const void *)self_attn_kernel<true>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kSmallLds * 4)));
-            GRX_HIP(hipFuncSetAttribute((const void *)self_attn_kernel<false>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(kSmallLds * 4)));
-        }
+        static GrxDeviceOnce once;  // set by the eager step that precedes any capture
+        GRX_HIP(grx_raise_lds(once, {(const void *)self_attn_kernel<true>, (const void *)self_attn_kernel<false>}, kSmallLds * 4));
     }
     const dim3 grid(nh, m->S * per);
     const size_t kv_stream = (size_t)hp.n_text_ctx * st;
