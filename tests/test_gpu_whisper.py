@@ -160,6 +160,29 @@ def test_prompt_passes_equal_steps(kern, orc, streams):
     assert _same(out[0][1], out[1][1])
 
 
+@pytest.mark.parametrize("streams,lengths", [(1, (3, 20, 33, 100, 256, 257)), (8, (3, 4, 5))])
+def test_prompt_rows_wide_model(kern, orc, streams, lengths):
+    """Rows of 1280 values, the second MLP product of 160 blocks (up to 32
+    rows carry its chain from one launch to the next), passes of one row to
+    256, the first MLP product's rounded GELU in every tile the sizes take:
+    logits and tokens of the same prompts token by token (PROMPT_ROWS=0)."""
+    from gorelaxor_amd.whisper import WhisperDecoder
+
+    hp = dict(WHISPER_TINY_TEST, n_state=1280, n_head=20, n_layer=1, n_text_ctx=320)
+    dec = WhisperDecoder(hp, whisper_model(hp, seed=6), streams=streams)
+    for k in range(streams):
+        dec.set_encoder_output_stream(k, encoder_output(hp, seed=60 + k))
+    for n in lengths:
+        prompts = np.random.default_rng(n).integers(0, hp["n_vocab"], (streams, n)).astype(np.int32)
+        out = []
+        for rows in (1, 0):
+            with kern.tuned(PROMPT_ROWS=rows):
+                first = dec.greedy_streams(prompts, 3) if streams > 1 else dec.greedy(prompts[0].tolist(), 3)
+                out.append((np.asarray(first), np.stack([dec.logits(k) for k in range(streams)])))
+        assert np.array_equal(out[0][0], out[1][0]), n
+        assert _same(out[0][1], out[1][1]), n
+
+
 def test_context_limit_and_errors(kern, orc):
     from gorelaxor_amd import GrxError
     from gorelaxor_amd.whisper import WhisperDecoder
