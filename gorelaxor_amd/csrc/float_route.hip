@@ -422,3 +422,28 @@ grx_status grx_float_rows_f32(hipStream_t st, const float *x, const float *w, co
     }
     return GRX_OK;
 }
+
+extern "C" grx_status grx_debug_rows_f32(grx_ctx *ctx, float *dst, const float *x, int m, const float *w, int rows,
+                                         int cols, const float *bias) {
+    if (!ctx || m < 0 || rows < 0 || cols < 0 || ((!dst || !x || !w) && m > 0 && rows > 0))
+        return grx_fail(GRX_EINVAL, "grx_debug_rows_f32: NULL argument or negative size");
+    if (m == 0 || rows == 0) return GRX_OK;
+    const size_t wb = (size_t)rows * cols * 4, xb = (size_t)m * cols * 4, yb = (size_t)m * rows * 4;
+    const size_t bb = bias ? (size_t)rows * 4 : 0;
+    auto up = [](size_t v) { return (v + 255) / 256 * 256; };
+    void *buf;
+    grx_status s = grx_ctx_scratch(ctx, up(wb) + up(xb) + up(yb) + up(bb) + 256, &buf);
+    if (s != GRX_OK) return s;
+    char *p = static_cast<char *>(buf);
+    float *dw = reinterpret_cast<float *>(p), *dx = reinterpret_cast<float *>(p + up(wb));
+    float *dy = reinterpret_cast<float *>(p + up(wb) + up(xb));
+    float *dbias = bias ? reinterpret_cast<float *>(p + up(wb) + up(xb) + up(yb)) : nullptr;
+    GRX_HIP(hipSetDevice(ctx->device));
+    GRX_HIP(hipMemcpyAsync(dw, w, wb, hipMemcpyHostToDevice, ctx->stream));
+    GRX_HIP(hipMemcpyAsync(dx, x, xb, hipMemcpyHostToDevice, ctx->stream));
+    if (bias) GRX_HIP(hipMemcpyAsync(dbias, bias, bb, hipMemcpyHostToDevice, ctx->stream));
+    if ((s = grx_float_rows_f32(ctx->stream, dx, dw, dbias, dy, 1, m, rows, cols)) != GRX_OK) return s;
+    GRX_HIP(hipMemcpyAsync(dst, dy, yb, hipMemcpyDeviceToHost, ctx->stream));
+    GRX_HIP(hipStreamSynchronize(ctx->stream));
+    return GRX_OK;
+}

@@ -154,6 +154,20 @@ def LinearF32(dst: np.ndarray, x: np.ndarray, w: np.ndarray, rows: int, cols: in
               cols, _ptr(None if bias is None else np.ascontiguousarray(bias, np.float32)))
 
 
+def rows_f32(dst: np.ndarray, x: np.ndarray, w: np.ndarray, bias=None, ctx: Context | None = None) -> None:
+    """kern.Linear of x's rows on a float32 weight through the launches of the
+    models' float32 products (grx_debug_rows_f32), host arrays."""
+    ctx = ctx or default_context()
+    x, w = np.ascontiguousarray(x, np.float32), np.ascontiguousarray(w, np.float32)
+    (m, k), n = x.shape, w.shape[0]
+    if w.shape[1] != k or dst.dtype != np.float32 or dst.shape != (m, n) or not dst.flags.c_contiguous:
+        raise IndexError("kern: rows and weight of other shapes than dst")
+    if bias is not None and bias.size < n:
+        raise IndexError("kern: bias shorter than the weight's rows")
+    _lib.call("grx_debug_rows_f32", ctx.handle, _ptr(dst), _ptr(x), m, _ptr(w), n, k,
+              _ptr(None if bias is None else np.ascontiguousarray(bias, np.float32)))
+
+
 def ToQ8(v: np.ndarray, rows: int, cols: int, ctx: Context | None = None) -> np.ndarray:
     """Weight.ToQ8 of an F32 matrix (kern.go:136-170) on the GPU: the Q8_0 bytes."""
     ctx = ctx or default_context()

@@ -743,6 +743,13 @@ long long grx_debug_alloc_countdown(void);
  * already captured keeps the kernels it captured.  GRX_EINVAL for an
  * unknown name. */
 grx_status grx_debug_tune(const char *name, int value);
+/* kern.Linear of m rows x [m][cols] on a float32 weight w [rows][cols]
+ * (gemm.go:116-259: k6x16 for the rows in whole groups of six when there are
+ * more than 16, gemvRows for the rest) into dst [m][rows], bias nullable: the
+ * launches the models' float32 convolutions and linears run, on host buffers,
+ * for tests of values no model's tensors hold. */
+grx_status grx_debug_rows_f32(grx_ctx *ctx, float *dst, const float *x, int m, const float *w, int rows, int cols,
+                              const float *bias);
 
 #ifdef __cplusplus
 }

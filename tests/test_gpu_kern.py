@@ -490,3 +490,54 @@ def test_linear_f32_bit_exact(kern, orc, n, k):
         kern.LinearF32(got, x, w, n, k, b)
         want = orc.matmul_f32(x[None], w, b)[0]
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (n, k, b is None)
+
+
+def _float_cases(rng, kind, m, n, k):
+    """x [m][k] and w [n][k] whose products' chains meet what `kind` names."""
+    x, w = rng.standard_normal((m, k)), rng.standard_normal((n, k))
+    if kind == "subnormal":  # sums and products down to and below 2^-149
+        x, w = x * 2.0 ** rng.integers(-90, -60, (m, k)), w * 2.0 ** rng.integers(-80, -60, (n, k))
+    if kind == "subnormal_inputs":
+        x, w = x * 2.0 ** rng.integers(-149, -132, (m, k)), w * 2.0 ** rng.integers(-2, 4, (n, k))
+    if kind == "cancel":  # exponents far apart and exact cancellations
+        x, w = x * 2.0 ** rng.integers(-20, 20, (m, k)), w * 2.0 ** rng.integers(-20, 20, (n, k))
+        x[:, 1::2], w[:, 1::2] = x[:, ::2][:, :k // 2], -w[:, ::2][:, :k // 2]
+    if kind == "overflow":  # sums past the largest float, and back from infinity (NaN)
+        x, w = x * 2.0 ** rng.integers(55, 65, (m, k)), w * 2.0 ** rng.integers(60, 64, (n, k))
+    with np.errstate(over="ignore"):
+        x, w = x.astype(np.float32), w.astype(np.float32)
+    if kind == "zeros":  # sums that stay at a zero, of either sign
+        x[rng.random((m, k)) < 0.9] = 0.0
+        w[rng.random((n, k)) < 0.5] = -0.0
+        x[rng.random((m, k)) < 0.5] *= -1
+        x[::3] = -0.0
+        w[::5] = -0.0
+    if kind == "specials":
+        for a in (x, w):
+            for v in (np.inf, -np.inf, np.nan):
+                a[rng.integers(0, a.shape[0], 3), rng.integers(0, k, 3)] = v
+    return x, w
+
+
+@pytest.mark.parametrize("kind", ["subnormal", "subnormal_inputs", "cancel", "overflow", "zeros", "specials"])
+@pytest.mark.parametrize("m,n,k", [(50, 20, 70), (64, 32, 515), (70, 67, 300), (18, 130, 129), (2101, 1000, 37),
+                                   (7, 20, 70)])
+def test_rows_f32_unusual_values(kern, orc, m, n, k, kind):
+    """The float32 matrix-core rows (narrow, 32 x 32 and 64 x 64 tiles, K that
+    ends within a pass and past the chunk of 256) and their gemvRows rest, on
+    chains that meet subnormal numbers, zeros of either sign, cancellation,
+    overflow, infinities and NaN: the oracle's fused multiply-add chains bit
+    for bit (a NaN where it has one).  The prompt's cross-attention runs the
+    same instruction."""
+    rng = np.random.default_rng(m + n + k)
+    x, w = _float_cases(rng, kind, m, n, k)
+    bias = np.where(rng.random(n) < 0.5, np.float32(-0.0), np.float32(2.0 ** -140 if "sub" in kind else 1.0))
+    for b in (None, bias.astype(np.float32)):
+        got = np.zeros((m, n), np.float32)
+        kern.rows_f32(got, x, w, b)
+        want = orc.matmul_f32(x, w, b)
+        assert _bits_equal_nan(got, want), _report(got, want)
+        if kind.startswith("subnormal"):
+            assert (np.abs(want[want != 0]) < 2.0 ** -126).any()
+        if kind in ("overflow", "specials"):
+            assert np.isinf(want).any() or np.isnan(want).any()
