@@ -183,6 +183,22 @@ def test_prompt_rows_wide_model(kern, orc, streams, lengths):
         assert _same(out[0][1], out[1][1]), n
 
 
+@pytest.mark.parametrize("kernel", [1, 2, 3])
+@pytest.mark.parametrize("n", [5, 70])
+def test_prompt_rows_each_product_kernel(kern, orc, n, kernel):
+    """A prompt's products, the rounded GELU among them, on the register walk
+    (GEMM_KERNEL=1), the K-split kernel (2) and the LDS-staged tiles (3):
+    the last row's logits and the next step's, bit for bit."""
+    hp = dict(WHISPER_TINY_TEST, n_text_ctx=96)
+    ref, dec = _pair(orc, hp, seed=n)
+    toks = np.random.default_rng(n).integers(0, hp["n_vocab"], n).tolist()
+    with kern.tuned(GEMM_KERNEL=kernel):
+        for m in (toks, toks[:1]):
+            lr = ref.decode(m)
+            lg, _ = dec.decode(m)
+            assert _same(lg, lr), f"{len(m)} at {dec.pos}: max |diff| {np.abs(lg - lr).max()}"
+
+
 def test_context_limit_and_errors(kern, orc):
     from gorelaxor_amd import GrxError
     from gorelaxor_amd.whisper import WhisperDecoder
