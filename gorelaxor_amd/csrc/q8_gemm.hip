@@ -16,9 +16,8 @@
 // MFMAs sharing the A fragment); a workgroup of four waves covers 64 x 64.
 // Per block a lane loads 8 bytes of A, 4 x 8 bytes of B (the weight tile
 // layout keeps each row's 32 bytes in two 16-byte halves), four weight scales
-// and four activation scales.  The per-output fold (convert, multiply, fma; two
-// fmas in the LDS-staged kernel:
-// 2-3 VALU ops per output per block) is the bound, not the MFMA: exact
+// and four activation scales.  The per-output fold (convert, multiply, fma:
+// 3 VALU ops per output per block) is the bound, not the MFMA: exact
 // per-block scaling costs that much vector work per 32 multiply-adds.
 #include <cstdint>
 #include <cstdlib>
@@ -884,17 +883,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p, size_t
 // of once per wave.
 //
 // Bound by the fold, c = fma(f32(s_b) * dw_b, da_b, c) per output and block
-// in order, on the vector units.  Its convert and multiply are one fma here:
-// the MFMA adds the int32 sum s to the bits of M = 1.5 * 2^23, which reads as
-// the float M + s exactly (|s| <= 2^19), and fma(M + s, dw, -M dw) rounds
-// s dw once: M dw is exact (dw has float16's 11 significant bits, M has two),
-// so the bits are the product's.  Two cases differ: an infinite dw (NaN
-// instead of an infinity) and the sign of a zero product of a zero or
-// negative dw.  A workgroup that meets such a scale takes the convert and
-// the multiply from there on.
-constexpr uint32_t kFoldMagic = 0x4B400000u;  // the bits of M
-constexpr float kFoldM = 12582912.0f;
-
+// in order, on the vector units: convert, multiply, fma.  (Convert and
+// multiply as one fma of the sum's bits behind 1.5 * 2^23 keeps the bits for
+// positive finite scales and was 1-9 % faster in the narrow tiles with those
+// alone; the second form that a zero, negative or infinite scale needs, as
+// all-zero blocks have, cost more than that: 2016 x 1024 x 4096 with a zero
+// scale in 10,000 52.0 us against 46.0 with three operations, 64 x 4096 x 4096
+// 20.5 against 16.4.)
 template <int WM, int WN, int FR, int FC, int CB>
 struct LdsTile {
     static constexpr int TM = 16 * FR * WM, TN = 16 * FC * WN, NT = 64 * WM * WN;
@@ -922,7 +917,6 @@ __global__ __launch_bounds__(64 * WM *WN, FR *FC == 4 ? 4 : 2) void gemm_q8_lds_
     constexpr int NT = T::NT;
     static_assert(FC == 2 || (!epi_rounds(EPI) && EPI != GRX_GEMM_GLU), "whole 32-column groups");
     __shared__ __align__(16) uint8_t lds[2 * T::kBuf];
-    __shared__ int odd;  // a scale that is not positive and finite has come
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WN, wn = wave % WN;  // wave rows 16 FR wm.., columns 16 FC wn..
@@ -941,7 +935,6 @@ __global__ __launch_bounds__(64 * WM *WN, FR *FC == 4 ? 4 : 2) void gemm_q8_lds_
     const int mb = (byrow ? hi : lo) * T::TM, nc = (byrow ? lo : hi) * T::TN;  // activation rows mb.., weight rows nc..
     const int K = nb * GRX_QK;
     const int li = lane & 15, lk = lane >> 4;
-    if (tid == 0) odd = 0;
 
     // ---- the copy of blocks [b0, b0+CB) into registers, then LDS, in pieces
     // of 16 bytes and single scales.  Nothing branches: a load whose result
@@ -1007,19 +1000,16 @@ __global__ __launch_bounds__(64 * WM *WN, FR *FC == 4 ? 4 : 2) void gemm_q8_lds_
 #pragma unroll
         for (int h = 0; h < NB; ++h)
             *reinterpret_cast<v4u *>(base + T::kA + 16 * ((tid + h * NT) % kBpc)) = S.b[h];
-        bool bad = false;
 #pragma unroll
         for (int h = 0; h < ND; ++h) {
             const int pc = (tid + h * NT) % kDpc;
             dl[pc] = grx_f16_to_f32(S.d[h]);
-            bad |= S.d[h] - 1u >= 0x7bffu && nc + pc % T::TN < rows;
         }
 #pragma unroll
         for (int h = 0; h < NS; ++h) {
             const int pc = (tid + h * NT) % kSpc;
             sl[(pc % CB) * T::TM + pc / CB] = S.s[h];
         }
-        if (bad) odd = 1;
     };
 
     float c[FR][FC][4];  // [row frag][column frag][r]
@@ -1059,8 +1049,8 @@ __global__ __launch_bounds__(64 * WM *WN, FR *FC == 4 ? 4 : 2) void gemm_q8_lds_
     struct Dots {
         v4i d[FR][FC];
     };
-    auto products = [&](const Ops &o, int z0) {
-        const v4i z = {z0, z0, z0, z0};
+    auto products = [&](const Ops &o) {
+        const v4i z = {0, 0, 0, 0};
         Dots p;
 #pragma unroll
         for (int f = 0; f < FR; ++f)
@@ -1068,58 +1058,50 @@ __global__ __launch_bounds__(64 * WM *WN, FR *FC == 4 ? 4 : 2) void gemm_q8_lds_
             for (int g = 0; g < FC; ++g) p.d[f][g] = __builtin_amdgcn_mfma_i32_16x16x32_i8(o.a[f], o.b[g], z, 0, 0, 0);
         return p;
     };
-    auto fold = [&](const Ops &o, const Dots &p, auto plain) {
+    auto fold = [&](const Ops &o, const Dots &p) {
 #pragma unroll
-        for (int g = 0; g < FC; ++g) {
-            const float md = __fmul_rn(-kFoldM, o.dw[g]);
+        for (int g = 0; g < FC; ++g)
 #pragma unroll
-            for (int f = 0; f < FR; ++f) {
+            for (int f = 0; f < FR; ++f)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int d = p.d[f][g][r];
-                    const float t = decltype(plain)::value ? __fmul_rn((float)d, o.dw[g])
-                                                           : __fmaf_rn(__int_as_float(d), o.dw[g], md);
-                    c[f][g][r] = __fmaf_rn(t, o.da[f][r], c[f][g][r]);
-                }
-            }
-        }
+                for (int r = 0; r < 4; ++r)
+                    c[f][g][r] = __fmaf_rn(__fmul_rn((float)p.d[f][g][r], o.dw[g]), o.da[f][r], c[f][g][r]);
     };
     auto blocks = [&](int buf, int st) {
         const uint8_t *base = lds + buf * T::kBuf;
         const int ub = min(CB, nb - st * CB);
-        const bool slow = __builtin_amdgcn_readfirstlane(odd) != 0;
-        if (!slow && ub == CB) {
+        if (ub == CB) {
             if constexpr (FR * FC == 4) {
                 // block by block: registers for two workgroups a CU, whose
                 // waves overlap each other's reads, products and folds
 #pragma unroll
                 for (int u = 0; u < CB; ++u) {
                     const Ops o = read(base, u);
-                    fold(o, products(o, (int)kFoldMagic), std::false_type{});
+                    fold(o, products(o));
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
                 // a block's products are issued before the fold of the block
                 // before it, its operands read one block earlier still
                 Ops o0 = read(base, 0), o1 = read(base, 1);
-                Dots p = products(o0, (int)kFoldMagic);
+                Dots p = products(o0);
 #pragma unroll
                 for (int u = 0; u < CB; ++u) {
                     Ops o2;
                     Dots pn;
                     if (u + 2 < CB) o2 = read(base, u + 2);
-                    if (u + 1 < CB) pn = products(o1, (int)kFoldMagic);
-                    fold(o0, p, std::false_type{});
+                    if (u + 1 < CB) pn = products(o1);
+                    fold(o0, p);
                     o0 = o1;
                     o1 = o2;
                     p = pn;
                 }
             }
-        } else {
+        } else {  // a K that ends within a stage
 #pragma unroll 1
             for (int u = 0; u < ub; ++u) {
                 const Ops o = read(base, u);
-                fold(o, products(o, 0), std::true_type{});
+                fold(o, products(o));
             }
         }
     };
@@ -1127,7 +1109,6 @@ __global__ __launch_bounds__(64 * WM *WN, FR *FC == 4 ? 4 : 2) void gemm_q8_lds_
     Set s0, s1;
     gload(s0, 0);
     gload(s1, CB);
-    __syncthreads();  // odd is 0
     lstore(s0, 0);
     __syncthreads();
     int st = 0;

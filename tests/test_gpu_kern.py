@@ -336,8 +336,8 @@ def test_matmul_prequant_alignment(kern, orc, dev, m, n, k, off):
 def test_matmul_lds_unusual_scales(kern, m, n, scale):
     """Blocks whose scale is zero, negative, infinite, not a number, the
     least or the greatest one, among ordinary ones, and a bias of -0: the
-    LDS-staged product's one-fma scaling gives the bits of the K-split
-    kernel's convert and multiply (a NaN where that has one)."""
+    LDS-staged product gives the bits of the K-split kernel (a NaN where that
+    has one)."""
     rng = np.random.default_rng(scale + n)
     k = 32 * 20
     w8 = rng.integers(0, 256, (n, k // 32, 34), dtype=np.uint8)
