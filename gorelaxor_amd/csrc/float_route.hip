@@ -33,7 +33,7 @@ namespace {
 //
 // On the float32 matrix cores: v_mfma_f32_16x16x4_f32 adds its four products
 // to the accumulator one after another in k order with one rounding each,
-// which is four steps of the chain (checked bit for bit against fmaf chains,
+// which is four steps of the chain (tests hold it to fmaf chains bit for bit,
 // with subnormal sums, signed zeros, infinities and NaN).  A workgroup of
 // WR x WC waves computes 16 WR RF x 16 WC CF outputs, KC k's a pass through
 // LDS, double-buffered.  Within each 16 k's LDS holds k = 4s + l at place

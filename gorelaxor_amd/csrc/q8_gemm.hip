@@ -895,7 +895,9 @@ struct LdsTile {
     static constexpr int TM = 16 * FR * WM, TN = 16 * FC * WN, NT = 64 * WM * WN;
     // per buffer: A [TM rows][CB][32] bytes, rows kAr apart (16 bytes of
     // padding: a fragment's 8-byte reads of 16 rows and a row's 16-byte
-    // stores fall in distinct banks), B [CB][2 halves][TN][16], weight scales
+    // stores fall in distinct banks; the counters show 1.3 conflict cycles an
+    // LDS instruction in the 64 x 128 tile and 3.0-3.4 in the narrow ones,
+    // the activation scales' transposing stores among them), B [CB][2 halves][TN][16], weight scales
     // [CB][TN] f32, activation scales [CB][TM] f32
     static constexpr int kAr = CB * 32 + 16;
     static constexpr int kA = TM * kAr, kB = CB * 32 * TN, kD = CB * TN * 4, kS = CB * TM * 4;
@@ -1438,12 +1440,14 @@ template <int EPI>
 void launch_lds(hipStream_t st, const grx_weight *w, const int8_t *xq, const float *xs, int m, const float *bias,
                 const GemmOut &o) {
     // 64 x 128 tiles from 144 of them on (two in flight a CU fold fastest:
-    // 2016 x 4096 x 1024 44.5 us against 65 in 64 x 32; 160 tiles of 300 x
-    // 4096 x 1024 16.2 against 17.6, 128 of 1000 x 1024 x 1024 16.9 against
-    // 14.4).  Fewer leave CUs idle: 64 x 32 then (300 x 1024 x 4096, 40 wide
-    // tiles, 45 -> 22.8 us), or 32 x 32 where even those are at most 128
-    // (256 x 1024 x 1024 10.3 -> 9.0 us, 15.8 in 64 x 128).  Whole calls with
-    // the rounding launch.
+    // 2016 x 4096 x 1024 45.0 us against 65.5 in 64 x 32; 160 tiles of 300 x
+    // 4096 x 1024 15.6 against 17.1, 128 of 1000 x 1024 x 1024 15.5 against
+    // 13.3).  Fewer leave CUs idle: 64 x 32 then (300 x 1024 x 4096, 40 wide
+    // tiles, 39.6 against 23.4 us), or 32 x 32 where even those are at most
+    // 128 (256 x 1024 x 1024 9.7 against 9.1 us, 14.1 in 64 x 128).  The rule
+    // counts tiles and looks neither at K nor at rows past a tile's end: 96 x
+    // 5120 x 1280 takes 13.7 us where 32 x 32 tiles, three whole row groups,
+    // take 11.6.  Whole calls with the rounding launch.
     if (grx_ceil_div(m, 64) * grx_ceil_div(w->rows, 128) >= 144)
         launch_lds_tile<EPI, 2, 4, 2, 2, 4>(st, w, xq, xs, m, bias, o);
     else if (grx_ceil_div(m, 64) * grx_ceil_div(w->rows, 32) > 128)
@@ -1462,13 +1466,13 @@ void launch_lds(hipStream_t st, const grx_weight *w, const int8_t *xq, const flo
 // against 8.0 K-split; a forced GEMM_KERNEL keeps the matrix cores); the
 // LDS-staged tiles from 256 rows on, and from 33 where 64 x 32 tiles of the
 // output are 128 or more or the K-split kernel does not take the product
-// (calls with the rounding launch: 126 x 4096 x 1024 10.5 us against 12.3
-// K-split, 126 x 2048 x 1024 8.8 against 9.8, 240 x 1024 x 4096 17.6 against
-// 21.0, 48 x 4096 x 1024 8.9 against 9.8; with 64 tiles the K-split wins: 126
-// x 1024 x 4096 13.8 against 16.4; blocks in no groups of four: 33 x 4096 x
-// 1056 7.8 against 8.3 on the register walk, 255 x 16384 x 480 15.1 against
-// 24.0; more blocks than a K-split workgroup holds: 100 x 1280 x 5120 18.1
-// against 33.0, 40 x 64 x 4640 16.4 against 22.6); below that the K-split
+// (calls with the rounding launch: 126 x 4096 x 1024 9.7 us against 11.4
+// K-split, 126 x 2048 x 1024 9.1 against 9.2, 240 x 1024 x 4096 18.6 against
+// 20.7, 48 x 4096 x 1024 9.1 against 9.4; with 64 tiles the K-split wins: 126
+// x 1024 x 4096 13.1 against 16.9; blocks in no groups of four: 200 x 16384 x
+// 480 16.2 against 47.7 on the register walk; more blocks than a K-split
+// workgroup holds: 100 x 1280 x 5120 20.0 against 33.2, 64 x 1000 x 4640 18.2
+// against 26.9); below that the K-split
 // tiles with their activations staged through LDS (at 224 rows: 1024 x 4096
 // 17 us against 26 on the whole-K register walk); without the staging, the
 // K-split tiles up to 128 rows where the register walk had few tiles or a

@@ -782,9 +782,9 @@ __global__ __launch_bounds__(256) void argmax_finish_kernel(const unsigned long 
     if (tid == 0) *pos = *pos + (streams ? 1 : M);
 }
 
-// One thread per block: quantU8 of m rows (q8int.go:88-105), signed.
-// Eight lanes a block, 16 bytes a lane (a thread a block touched 64 lines a
-// load: 300 x 4096 4.9 us, 4.3 here).
+// quantU8 of m rows (q8int.go:88-105), signed: eight lanes a block, 16 bytes
+// a lane (a thread a block touched 64 lines a load: 300 x 4096 4.9 us, 4.3
+// here).
 __global__ __launch_bounds__(256) void quant_act_kernel(const float *__restrict__ x, int lda, int m, int nb,
                                                         int8_t *__restrict__ q, float *__restrict__ sc) {
     const int i = blockIdx.x * 32 + (threadIdx.x >> 3), l8 = threadIdx.x & 7;

@@ -67,9 +67,10 @@ __global__ __launch_bounds__(kThreads) void ln_quant_rows_kernel(const float *__
 }
 
 // Row r: x[r] = tokEmb.row(tok[r]) + decPos[*pos + r % per] (whisper/
-// decoder.go:42-46; `per` consecutive positions of each stream, 1 in a step; the embedding row widened from its Q8_0 tile layout,
-// d*q then + pos unfused), stored as the residual stream, then LayerNorm
-// and rounding as above.
+// decoder.go:42-46; `per` consecutive positions of each stream, 1 in a step;
+// the embedding row widened from its Q8_0 tile layout, d*q then + pos
+// unfused), stored as the residual stream, then LayerNorm and rounding as
+// above.
 __global__ __launch_bounds__(kThreads) void embed_ln_quant_kernel(
     const int *__restrict__ tok, const int *__restrict__ pos, const int8_t *__restrict__ emb_qs,
     const uint16_t *__restrict__ emb_ds, int nb, const float *__restrict__ pos_emb, float *__restrict__ x,
